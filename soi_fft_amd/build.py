@@ -17,7 +17,9 @@ LIB = os.path.join(HERE, "libsoi_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = os.environ.get("SOI_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["soi_kernels.hip", "soi_filter.hip", "soi_fft.hip"]
+HIP_SOURCES = ["soi_filter.hip", "soi_kernels.hip", "soi_fft.hip", "soi_fft_cols64.hip",
+               "soi_fft_cols32.hip", "soi_fft_rows64.hip", "soi_fft_rows32.hip",
+               "soi_fft_long32.hip"]
 C_SOURCES = ["pfft.c", "compress_host.c", "harness.c"]
 DRIVER = os.path.join(HERE, "soi_test")   # command-line driver (soi_test.c), links the library
 

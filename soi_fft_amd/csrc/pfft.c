@@ -77,7 +77,6 @@ void soi_internal_set_error(int status, const char *msg)
 /* ------------------------------------------------------------------------------------------ */
 #define NSTAGE 4
 #define NTSLOT 64 /* timed calls kept for soi_stage_times */
-#define SOI_MAX_FFT_GROUPS 32
 typedef struct {
   int device;
   hipStream_t stream;
@@ -93,15 +92,16 @@ typedef struct {
   soi_c32_t *taps32, *post32, *twS32, *tw1_32, *tw2_32, *thi32, *tlo32;
   void *wt; /* complex64 MFMA filter: bf16 tap pieces */
   /* fft */
+  int fft_one;                     /* one pass, one segment per block (fft_single then too) */
+  int fft_long;                    /* complex64 of N >= 2^24: the passes of soi_fft_long32.hip */
   int fft_single, single_count, fft_reg;
-  int n1, n2, Tc, Tr, B1, lb1, clay;
-  /* register-FFT alternatives (column tile, column variant, row tile) and the one in use */
-  int nvar, var;
-  int vtab[16][3];
-  /* pass 1 writes 8-row tiles into tbuf (S*M_hat values) and pass 2 reads them (register
-   * path).  A buffer of the plan's own: a caller's gamma_tilde may be sized as the
-   * reference's per-rank work buffer. */
-  int tiled;
+  int n1, n2, Tc, Tr, B1, lb1;
+  int cvar, rvar;                  /* tile alternatives of the column and row pass in use */
+  int nvar, var;                   /* var = cvar + (column alternatives) * rvar */
+  /* complex64: pass 1 writes 8-row tiles into tbuf and pass 2 reads them (register path);
+   * Mt values per segment, n1 rounded up to whole tiles.  A buffer of the plan's own: a caller's
+   * gamma_tilde may be sized as the reference's per-rank work buffer. */
+  long Mt;
   void *tbuf;
   soi_c64_t *tw1, *tw2, *thi, *tlo;
   /* buffers */
@@ -122,12 +122,6 @@ typedef struct {
   int *h_vlc;
   int vlc_valid;
   hipStream_t last_stream; /* stream of the last compute call */
-  /* segment groups of the register FFT path: pass 1 of group g + 1 runs beside pass 2 of group
-   * g on a second stream, so that pass 2 reads pass 1's output while it is still in the
-   * last-level cache (fft_groups = 1: both passes over all segments, one launch each) */
-  int fft_groups;
-  hipStream_t stream2;
-  hipEvent_t gev[SOI_MAX_FFT_GROUPS + 2];
   /* timing: NSTAGE+1 events per call, in a ring of NTSLOT calls */
   int timing;
   long ncalls;          /* calls recorded since timing was enabled */
@@ -223,40 +217,13 @@ static int pick_tile(int n, long other, int cap)
   return 0;
 }
 
-/* Register-FFT alternatives that exist for (n1, n2): column tile 8 or 4 with its kernel
- * variant, row tile 8 or 4.  The planned choice is entry 0 of the table. */
-static void fft_variants(soi_plan_t *pl)
+/* Time of one register pass over n-point transforms (rows = 0: columns) in units of a pass at
+ * 4.9 TB/s of its own bytes: what the default tiles measured at 1.34 GB (see soi_fft.hpp). */
+static double pass_cost(long n, int rows, int f32)
 {
-  int cols[6][2], nc = 0, rows[2], nr = 0;
-  const int n1 = pl->n1, n2 = pl->n2;
-  const int c4 = n1 == 1024 || n1 == 1280 || n1 == 2048 || n1 == 2560;
-  cols[nc][0] = pl->Tc, cols[nc][1] = pl->clay, ++nc;
-  if (soik_fft_cols_short_tile(n1)) { /* short columns: one configuration */
-    pl->nvar = 1;
-    pl->vtab[0][0] = pl->Tc, pl->vtab[0][1] = pl->clay, pl->vtab[0][2] = pl->Tr;
-    pl->var = 0;
-    return;
-  }
-  if (n2 % 8 == 0 && !(pl->Tc == 8 && pl->clay == 0)) cols[nc][0] = 8, cols[nc][1] = 0, ++nc;
-  if (c4 && n2 % 4 == 0 && !(pl->Tc == 4 && pl->clay == 0)) cols[nc][0] = 4, cols[nc][1] = 0, ++nc;
-  if ((n1 == 2048 || n1 == 2560) && n2 % 8 == 0 && pl->clay != 1)
-    cols[nc][0] = 8, cols[nc][1] = 1, ++nc;
-  if (n1 == 2560 && n2 % 4 == 0 && pl->clay != 2 && nc < 5) cols[nc][0] = 4, cols[nc][1] = 2, ++nc;
-  if (n1 == 2560 && pl->f32 && n2 % 8 == 0 && pl->clay != 3 && nc < 6)
-    cols[nc][0] = 8, cols[nc][1] = 3, ++nc;
-  if (n1 == 2560 && !pl->f32 && n2 % 4 == 0 && pl->clay != 4 && nc < 6)
-    cols[nc][0] = 4, cols[nc][1] = 4, ++nc;
-  rows[nr++] = pl->Tr;
-  if (pl->Tr != 8 && n2 != 2560 && n1 % 8 == 0) rows[nr++] = 8;
-  if (pl->Tr != 4 && (n2 == 1024 || n2 == 1280 || n2 == 2048 || n2 == 2560) && n1 % 4 == 0)
-    rows[nr++] = 4;
-  pl->nvar = 0;
-  for (int r = 0; r < nr; ++r)
-    for (int c = 0; c < nc; ++c) {
-      int *v = pl->vtab[pl->nvar++];
-      v[0] = cols[c][0], v[1] = cols[c][1], v[2] = rows[r];
-    }
-  pl->var = 0;
+  if (rows && n > 2048) return 1.9; /* half as wide: 64-byte store runs */
+  if (f32) return rows ? (n <= 640 ? 1.03 : n <= 1280 ? 1.5 : 1.4) : n <= 640 ? 1.07 : n <= 1280 ? 1.23 : 1.35;
+  return rows ? (n <= 640 ? 0.98 : n <= 1280 ? 1.12 : 1.2) : n <= 1280 ? 1.0 : 1.16;
 }
 
 static int plan_fft(soi_plan_t *pl)
@@ -267,33 +234,37 @@ static int plan_fft(soi_plan_t *pl)
     set_err(SOI_ERR_ARGS, "M_hat=%ld is not of the form 2^a 3^b 5^c", Mh);
     return -1;
   }
-  if (Mh + 1 <= CAP) {
-    pl->nvar = 1;
-    pl->var = 0;
-    pl->fft_single = 1;
-    pl->single_count = (int)(CAP / (Mh + 1));
-    if (pl->single_count > pl->S) pl->single_count = (int)pl->S;
-    if (pl->single_count < 1) pl->single_count = 1;
+  pl->nvar = 1;
+  pl->fft_long = pl->f32 && pl->N >= 1L << 24;
+  if (!pl->fft_long && Mh < INT_MAX && soik_fft_reg_supported((int)Mh, 2)) {
+    pl->fft_single = pl->fft_one = 1;
     return 0;
   }
-  pl->fft_single = 0;
-  /* register kernels: columns of n1 and rows of n2 both have one, 8-wide tiles on both sides */
+  /* two register passes: columns of n1 and rows of n2 points that both have kernels.  The split
+   * with the least measured pass times, scaled by what is padding in partial column and row tiles;
+   * about equal ones by the longer of the two lengths (the shorter it is, the more blocks a CU
+   * holds).  Long complex64 transforms keep their rule: the smallest longer length, then the
+   * longer column. */
   {
-    long best = LONG_MAX;
+    double best = 1e300;
     int bn1 = 0;
     /* SOI_FFT_N1 forces the column length (tuning) */
     const char *en = getenv("SOI_FFT_N1");
-    long force = en ? atol(en) : 0;
-    for (long n1 = 2; n1 <= 4096; ++n1) {
+    const long force = en ? atol(en) : 0;
+    for (long n1 = 2; n1 <= 2560; ++n1) {
       if (Mh % n1) continue;
-      long n2 = Mh / n1;
-      const int st = soik_fft_cols_short_tile((int)n1);
-      if (n2 % (st ? st : 8) || n2 > 4096) continue;
-      if (!soik_fft_reg_supported((int)n1, 0) || !soik_fft_reg_supported((int)n2, 1)) continue;
-      if (st && n1 % 8 && n2 != 256) continue; /* 10-wide rows exist for 256 points only */
-      long cost = (n1 > n2 ? n1 : n2);
+      const long n2 = Mh / n1;
+      if (n2 > 2560) continue;
+      if (pl->fft_long ? !soik_fft_long32_supported((int)n1) || !soik_fft_long32_supported((int)n2)
+                       : !soik_fft_reg_supported((int)n1, 0) || !soik_fft_reg_supported((int)n2, 1))
+        continue;
+      const long pc = (n2 + 7) / 8 * 8, pr = (n1 + 15) / 16 * 16;
+      const long longer = n1 > n2 ? n1 : n2;
+      double cost = pl->fft_long ? (double)longer
+                                 : pass_cost(n1, 0, pl->f32) * pc / n2 +
+                                       pass_cost(n2, 1, pl->f32) * pr / n1 + 1e-4 * longer;
       if (force == n1) cost = 0;
-      if (cost <= best) {   /* ties: the longer column */
+      if (cost < best || (cost == best && pl->fft_long)) {
         best = cost;
         bn1 = (int)n1;
       }
@@ -302,56 +273,22 @@ static int plan_fft(soi_plan_t *pl)
       pl->fft_reg = 1;
       pl->n1 = bn1;
       pl->n2 = (int)(Mh / bn1);
-      /* tile widths: 8 by default; SOI_FFT_TC / SOI_FFT_TR (4 or 8) override for tuning */
-      pl->Tc = pl->Tr = 8;
-      const char *ec = getenv("SOI_FFT_TC"), *er = getenv("SOI_FFT_TR");
-      if (ec && (atoi(ec) == 4 || atoi(ec) == 8)) pl->Tc = atoi(ec);
-      if (er && (atoi(er) == 4 || atoi(er) == 8)) pl->Tr = atoi(er);
-      if (pl->n2 % pl->Tc || pl->n1 % pl->Tr) pl->Tc = pl->Tr = 8;
-      if (pl->n2 == 2560) pl->Tr = 4; /* 2560-point rows exist with 4-wide tiles only */
-      const int stile = soik_fft_cols_short_tile(pl->n1);
-      if (stile) { /* short columns: their own tile width; rows 10-wide unless n1 % 8 == 0 */
-        pl->Tc = stile;
-        pl->Tr = pl->n1 % 8 ? 10 : 8;
-      }
-      /* column-pass kernel variant: 1 = one padded LDS run per sequence (8-wide tiles of 2048
-       * or 2560); 2 = one 4-wide block per CU with the whole register budget (2560: 20
-       * values per thread do not fit 1024-thread blocks); 4 = the same exchanging whole
-       * complex128 values in all 160 KiB of LDS (2560, the complex128 default: one round per
-       * exchange instead of a real and an imaginary one, 1.59 -> 1.51 ms at N = 2^27).
-       * Complex64 2560-point columns default to 4-wide tiles in two exchange groups, two
-       * blocks per CU (their whole-complex exchanges fit in 44 KB).  SOI_FFT_CVAR overrides
-       * for tuning */
-      const char *el = getenv("SOI_FFT_CVAR");
-      int cv = el && !stile ? atoi(el) : (pl->n1 == 2560 && !pl->f32 ? 4 : 0);
-      if (!el && !ec && pl->n1 == 2560 && pl->f32 && pl->n2 % 4 == 0) pl->Tc = 4;
-      pl->clay = 0;
-      if (cv == 1 && pl->Tc == 8 && (pl->n1 == 2048 || pl->n1 == 2560)) pl->clay = 1;
-      if (cv == 2 && pl->n1 == 2560) {
-        pl->clay = 2;
-        pl->Tc = 4;
-      }
-      if (cv == 3 && pl->n1 == 2560 && pl->f32) {
-        pl->clay = 3;
-        pl->Tc = 8;
-      }
-      if (cv == 4 && pl->n1 == 2560 && !pl->f32) {
-        pl->clay = 4;
-        pl->Tc = 4;
-      }
       int lb = 0;
       while ((1L << lb) * (1L << lb) < Mh) ++lb;
       pl->B1 = 1 << lb;
       pl->lb1 = lb;
-      /* tiled pass-1 output: the default for complex64 (measured faster there; for
-       * complex128 the tiled row pass spills and the split stores are slower), SOI_FFT_TILED
-       * overrides */
-      const char *et = getenv("SOI_FFT_TILED");
-      pl->tiled = (et ? atoi(et) != 0 : pl->f32) && pl->n1 % 8 == 0 &&
-                  soik_fft_rows_tiled_supported(pl->n2, pl->f32);
-      fft_variants(pl);
+      pl->Mt = (long)(pl->n1 + 7) / 8 * 8 * pl->n2;
+      pl->nvar = pl->fft_long ? 1 + (pl->n1 == 2560)
+                              : soik_fft_reg_variants(pl->n1, 0) * soik_fft_reg_variants(pl->n2, 1);
       return 0;
     }
+  }
+  if (Mh + 1 <= CAP) {
+    pl->fft_single = 1;
+    pl->single_count = (int)(CAP / (Mh + 1));
+    if (pl->single_count > pl->S) pl->single_count = (int)pl->S;
+    if (pl->single_count < 1) pl->single_count = 1;
+    return 0;
   }
   /* generic LDS kernels: n1 x n2 = Mh, both smooth, column tile Tc >= 2 and row tile Tr >= 2
    * preferred; minimise max(n1, n2) with n1 a power of two when possible */
@@ -382,9 +319,6 @@ static int plan_fft(soi_plan_t *pl)
   pl->n2 = bn2;
   pl->Tc = bTc;
   pl->Tr = bTr;
-  pl->nvar = 1;
-  pl->var = 0;
-  pl->vtab[0][0] = bTc, pl->vtab[0][1] = 0, pl->vtab[0][2] = bTr;
   int b1 = 1, lb = 0;
   while ((long)b1 * b1 < Mh) b1 <<= 1, ++lb;
   pl->B1 = b1;
@@ -427,9 +361,6 @@ static void free_plan(soi_plan_t *pl)
   for (int c = 0; c < NTSLOT; ++c)
     for (int e = 0; e <= NSTAGE; ++e)
       if (pl->ev[c][e]) (void)hipEventDestroy(pl->ev[c][e]);
-  for (int e = 0; e < SOI_MAX_FFT_GROUPS + 2; ++e)
-    if (pl->gev[e]) (void)hipEventDestroy(pl->gev[e]);
-  if (pl->stream2) (void)hipStreamDestroy(pl->stream2);
   if (pl->stream) (void)hipStreamDestroy(pl->stream);
   free(pl);
 }
@@ -510,19 +441,6 @@ void init_soi_descriptor(soi_desc_t *d, MPI_Comm comm, cfft_size_t k)
   pl->f32 = d->precision == SOI_PREC_FP32;
   if (plan_filter(pl, d->window_mode) || plan_fft(pl)) goto fail_quiet;
   HIPCHK(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking));
-  {
-    /* SOI_FFT_GROUPS: segment groups of the two-stream FFT schedule (a divisor of S) */
-    const char *eg = getenv("SOI_FFT_GROUPS");
-    int ng = eg ? atoi(eg) : 1;
-    if (ng < 1 || ng > SOI_MAX_FFT_GROUPS || S % ng || !pl->fft_reg) ng = 1;
-    pl->fft_groups = ng;
-    if (ng > 1) {
-      HIPCHK(hipStreamCreateWithFlags(&pl->stream2, hipStreamNonBlocking));
-      for (int e = 0; e < ng + 2; ++e)
-        HIPCHK(hipEventCreateWithFlags(&pl->gev[e], hipEventDisableTiming));
-    }
-  }
-
   /* segment boundaries p*k (pfft.c:144-147) */
   d->segmentBoundaries = (int *)malloc(sizeof(int) * (d->P + 1));
   for (int p = 0; p <= d->P; ++p) d->segmentBoundaries[p] = p * (int)k;
@@ -565,12 +483,12 @@ void init_soi_descriptor(soi_desc_t *d, MPI_Comm comm, cfft_size_t k)
       }
       pl->owns_at = 1;
     }
-    if (pl->tiled) {
-      hipError_t e = hipMalloc(&pl->tbuf, (size_t)S * pl->Mh * esz);
+    if (pl->fft_reg && pl->f32) {
+      hipError_t e = hipMalloc(&pl->tbuf, (size_t)S * pl->Mt * esz);
       if (e != hipSuccess) {
         pl->tbuf = NULL;
         set_err(SOI_ERR_ALLOC, "Failed to allocate the FFT tile buffer (%zu bytes): %s",
-                (size_t)S * pl->Mh * esz, hipGetErrorString(e));
+                (size_t)S * pl->Mt * esz, hipGetErrorString(e));
         goto fail_quiet;
       }
     }
@@ -769,50 +687,33 @@ fail:
 
 static int run_fft_f32(soi_desc_t *d, soi_plan_t *pl, soi_c32_t *X, SoiBatch b, hipStream_t st)
 {
-  soi_c32_t *at = (soi_c32_t *)pl->at;
+  soi_c32_t *at = (soi_c32_t *)pl->at, *tb = (soi_c32_t *)pl->tbuf;
   const soi_c64_t *winv = pl->winv;
+  const int S = (int)pl->S;
   if (pl->fft_single) {
     mark(pl, 2, st);
-    KCHK(soik_fft_single_f32(at, X, pl->tw1_32, winv, pl->Mh, pl->M, (int)pl->S,
-                             pl->single_count, b, st));
+    if (pl->fft_one)
+      KCHK(soik_fft_one_f32(at, X, pl->tw1_32, winv, (int)pl->Mh, pl->M, S, b, st));
+    else
+      KCHK(soik_fft_single_f32(at, X, pl->tw1_32, winv, pl->Mh, pl->M, S, pl->single_count, b, st));
     mark(pl, 3, st);
+  } else if (pl->fft_long && pl->fft_reg) {
+    KCHK(soik_fft_long32_cols(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
+                              S, pl->cvar, tb, b, st));
+    mark(pl, 3, st);
+    KCHK(soik_fft_long32_rows(tb, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Mh, pl->M, S, b, st));
   } else if (pl->fft_reg) {
-    soi_c32_t *gt = pl->tiled ? (soi_c32_t *)pl->tbuf : NULL;
-    const int ng = b.n > 0 ? 1 : pl->fft_groups, G = (int)pl->S / ng;
-    hipStream_t s2 = ng > 1 ? pl->stream2 : st;
-    if (ng > 1) {
-      HIPCHK(hipEventRecord(pl->gev[0], st));
-      HIPCHK(hipStreamWaitEvent(s2, pl->gev[0], 0));
-    }
-    for (int g = 0; g < ng; ++g) {
-      const long so = (long)g * G;
-      KCHK(soik_fft_cols_reg_f32(at + so * pl->Mh, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1,
-                                 pl->n2, pl->lb1, pl->Mh, G, pl->Tc, pl->clay,
-                                 gt ? gt + so * pl->Mh : NULL, b, st));
-      if (ng > 1) {
-        HIPCHK(hipEventRecord(pl->gev[1 + g], st));
-        HIPCHK(hipStreamWaitEvent(s2, pl->gev[1 + g], 0));
-      } else {
-        mark(pl, 3, st);
-      }
-      if (gt)
-        KCHK(soik_fft_rows_tiled_f32(gt + so * pl->Mh, X + so * pl->M, pl->tw2_32, winv, pl->n1,
-                                     pl->n2, pl->Mh, pl->M, G, b, s2));
-      else
-        KCHK(soik_fft_rows_reg_f32(at + so * pl->Mh, X + so * pl->M, pl->tw2_32, winv, pl->n1,
-                                   pl->n2, pl->Mh, pl->M, G, pl->Tr, b, s2));
-    }
-    if (ng > 1) {
-      HIPCHK(hipEventRecord(pl->gev[ng + 1], s2));
-      HIPCHK(hipStreamWaitEvent(st, pl->gev[ng + 1], 0));
-      mark(pl, 3, st);
-    }
+    KCHK(soik_fft_cols_f32(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
+                           S, pl->cvar, tb, pl->Mt, b, st));
+    mark(pl, 3, st);
+    KCHK(soik_fft_rows_f32(tb, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Mt, pl->M, S, pl->rvar, b,
+                           st));
   } else {
     KCHK(soik_fft_col_f32(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->Tc, pl->B1,
-                          pl->Mh, (int)pl->S, b, st));
+                          pl->Mh, S, b, st));
     mark(pl, 3, st);
-    KCHK(soik_fft_row_f32(at, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Tr, pl->Mh, pl->M,
-                          (int)pl->S, b, st));
+    KCHK(soik_fft_row_f32(at, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Tr, pl->Mh, pl->M, S, b,
+                          st));
   }
   return 0;
 fail:
@@ -824,48 +725,25 @@ static int run_fft(soi_desc_t *d, soi_plan_t *pl, void *Xv, SoiBatch b, hipStrea
   if (pl->f32) return run_fft_f32(d, pl, (soi_c32_t *)Xv, b, st);
   soi_c64_t *X = (soi_c64_t *)Xv;
   soi_c64_t *at = (soi_c64_t *)pl->at;
+  const int S = (int)pl->S;
   if (pl->fft_single) {
     mark(pl, 2, st);
-    KCHK(soik_fft_single(at, X, pl->tw1, pl->winv, pl->Mh, pl->M, (int)pl->S,
-                         pl->single_count, b, st));
+    if (pl->fft_one)
+      KCHK(soik_fft_one(at, X, pl->tw1, pl->winv, (int)pl->Mh, pl->M, S, b, st));
+    else
+      KCHK(soik_fft_single(at, X, pl->tw1, pl->winv, pl->Mh, pl->M, S, pl->single_count, b, st));
     mark(pl, 3, st);
   } else if (pl->fft_reg) {
-    soi_c64_t *gt = pl->tiled ? (soi_c64_t *)pl->tbuf : NULL;
-    const int ng = b.n > 0 ? 1 : pl->fft_groups, G = (int)pl->S / ng;
-    hipStream_t s2 = ng > 1 ? pl->stream2 : st;
-    if (ng > 1) {
-      HIPCHK(hipEventRecord(pl->gev[0], st));
-      HIPCHK(hipStreamWaitEvent(s2, pl->gev[0], 0));
-    }
-    for (int g = 0; g < ng; ++g) {
-      const long so = (long)g * G;
-      KCHK(soik_fft_cols_reg(at + so * pl->Mh, pl->tw1, pl->thi, pl->tlo, pl->n1, pl->n2,
-                             pl->lb1, pl->Mh, G, pl->Tc, pl->clay, gt ? gt + so * pl->Mh : NULL,
-                             b, st));
-      if (ng > 1) {
-        HIPCHK(hipEventRecord(pl->gev[1 + g], st));
-        HIPCHK(hipStreamWaitEvent(s2, pl->gev[1 + g], 0));
-      } else {
-        mark(pl, 3, st);
-      }
-      if (gt)
-        KCHK(soik_fft_rows_tiled(gt + so * pl->Mh, X + so * pl->M, pl->tw2, pl->winv, pl->n1,
-                                 pl->n2, pl->Mh, pl->M, G, b, s2));
-      else
-        KCHK(soik_fft_rows_reg(at + so * pl->Mh, X + so * pl->M, pl->tw2, pl->winv, pl->n1,
-                               pl->n2, pl->Mh, pl->M, G, pl->Tr, b, s2));
-    }
-    if (ng > 1) {
-      HIPCHK(hipEventRecord(pl->gev[ng + 1], s2));
-      HIPCHK(hipStreamWaitEvent(st, pl->gev[ng + 1], 0));
-      mark(pl, 3, st);
-    }
-  } else {
-    KCHK(soik_fft_col(at, pl->tw1, pl->thi, pl->tlo, pl->n1, pl->n2, pl->Tc, pl->B1, pl->Mh,
-                      (int)pl->S, b, st));
+    KCHK(soik_fft_cols(at, pl->tw1, pl->thi, pl->tlo, pl->n1, pl->n2, pl->lb1, pl->Mh, S, pl->cvar,
+                       NULL, 0, b, st));
     mark(pl, 3, st);
-    KCHK(soik_fft_row(at, X, pl->tw2, pl->winv, pl->n1, pl->n2, pl->Tr,
-                      pl->Mh, pl->M, (int)pl->S, b, st));
+    KCHK(soik_fft_rows(at, X, pl->tw2, pl->winv, pl->n1, pl->n2, pl->Mh, pl->M, S, pl->rvar, b,
+                       st));
+  } else {
+    KCHK(soik_fft_col(at, pl->tw1, pl->thi, pl->tlo, pl->n1, pl->n2, pl->Tc, pl->B1, pl->Mh, S, b,
+                      st));
+    mark(pl, 3, st);
+    KCHK(soik_fft_row(at, X, pl->tw2, pl->winv, pl->n1, pl->n2, pl->Tr, pl->Mh, pl->M, S, b, st));
   }
   return 0;
 fail:
@@ -1018,9 +896,9 @@ int soi_set_fft_variant(soi_desc_t *d, int v)
   }
   pl->var = v;
   if (pl->fft_reg) {
-    pl->Tc = pl->vtab[v][0];
-    pl->clay = pl->vtab[v][1];
-    pl->Tr = pl->vtab[v][2];
+    const int nc = pl->fft_long ? pl->nvar : soik_fft_reg_variants(pl->n1, 0);
+    pl->cvar = v % nc;
+    pl->rvar = v / nc;
   }
   return 0;
 }
@@ -1142,8 +1020,7 @@ static int same_shape(const soi_desc_t *a, const soi_desc_t *b)
 static int same_plan(const soi_desc_t *a, const soi_desc_t *b)
 {
   const soi_plan_t *pa = (const soi_plan_t *)a->plan, *pb = (const soi_plan_t *)b->plan;
-  return same_shape(a, b) && pa->var == pb->var && pa->tiled == pb->tiled &&
-         pa->Tc == pb->Tc && pa->Tr == pb->Tr && pa->clay == pb->clay &&
+  return same_shape(a, b) && pa->var == pb->var && pa->n1 == pb->n1 &&
          (pa->fa.wt != NULL) == (pb->fa.wt != NULL);
 }
 

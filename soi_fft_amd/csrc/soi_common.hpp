@@ -240,9 +240,8 @@ __device__ __forceinline__ void lds_barrier()
 // same XCD and its L2.
 __device__ __forceinline__ int xcd_remap(int bid, int nblocks)
 {
-  const int NX = 8;
-  if (nblocks % NX) return bid;
-  return (bid % NX) * (nblocks / NX) + bid / NX;
+  const int NX = 8, per = nblocks / NX, rem = nblocks % NX, x = bid % NX;
+  return x * per + (x < rem ? x : rem) + bid / NX;
 }
 
 }  // namespace soi

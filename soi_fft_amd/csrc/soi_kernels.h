@@ -70,28 +70,34 @@ int soik_fft_col_f32(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi
 int soik_fft_row_f32(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
                      const soi_c64_t *winv, int n1, int n2, int Tr, long Mh, long M, int S,
                      SoiBatch b, hipStream_t st);
+/* register FFT (soi_fft.hpp): columns (rows = 0), rows (1) or whole segments (2) of L points */
 int soik_fft_reg_supported(int L, int rows);
-int soik_fft_cols_short_tile(int L);
-int soik_fft_cols_reg(soi_c64_t *data, const soi_c64_t *tw1, const soi_c64_t *thi,
-                      const soi_c64_t *tlo, int n1, int n2, int lb1, long Mh, int S, int T,
-                      int layout, soi_c64_t *tout, SoiBatch b, hipStream_t st);
-int soik_fft_rows_reg(const soi_c64_t *data, soi_c64_t *X, const soi_c64_t *tw2,
-                      const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S, int T,
+int soik_fft_reg_variants(int L, int rows);
+int soik_fft_cols(soi_c64_t *data, const soi_c64_t *tw1, const soi_c64_t *thi,
+                  const soi_c64_t *tlo, int n1, int n2, int lb1, long Mh, int S, int variant,
+                  soi_c64_t *tout, long Mt, SoiBatch b, hipStream_t st);
+int soik_fft_rows(const soi_c64_t *data, soi_c64_t *X, const soi_c64_t *tw2,
+                  const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S, int variant,
+                  SoiBatch b, hipStream_t st);
+int soik_fft_one(const soi_c64_t *at, soi_c64_t *X, const soi_c64_t *tw, const soi_c64_t *winv,
+                 int L, long M, int S, SoiBatch b, hipStream_t st);
+/* complex64: columns write 8-row tiles (Mt values per segment) that the rows read */
+int soik_fft_cols_f32(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi,
+                      const soi_c32_t *tlo, int n1, int n2, int lb1, long Mh, int S, int variant,
+                      soi_c32_t *tout, long Mt, SoiBatch b, hipStream_t st);
+int soik_fft_rows_f32(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
+                      const soi_c64_t *winv, int n1, int n2, long Mt, long M, int S, int variant,
                       SoiBatch b, hipStream_t st);
-int soik_fft_cols_reg_f32(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi,
-                          const soi_c32_t *tlo, int n1, int n2, int lb1, long Mh, int S, int T,
-                          int layout, soi_c32_t *tout, SoiBatch b, hipStream_t st);
-/* pass 2 over pass 1's 8-row tiles (tout of the column pass) */
-int soik_fft_rows_tiled_supported(int n2, int f32);
-int soik_fft_rows_tiled(const soi_c64_t *data, soi_c64_t *X, const soi_c64_t *tw2,
-                        const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S,
-                        SoiBatch b, hipStream_t st);
-int soik_fft_rows_tiled_f32(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
-                            const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S,
-                            SoiBatch b, hipStream_t st);
-int soik_fft_rows_reg_f32(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
-                          const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S, int T,
-                          SoiBatch b, hipStream_t st);
+int soik_fft_one_f32(const soi_c32_t *at, soi_c32_t *X, const soi_c32_t *tw,
+                     const soi_c64_t *winv, int L, long M, int S, SoiBatch b, hipStream_t st);
+/* complex64 passes of long transforms (soi_fft_long32.hip) */
+int soik_fft_long32_supported(int L);
+int soik_fft_long32_cols(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi,
+                         const soi_c32_t *tlo, int n1, int n2, int lb1, long Mh, int S, int variant,
+                         soi_c32_t *tout, SoiBatch b, hipStream_t st);
+int soik_fft_long32_rows(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
+                         const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S, SoiBatch b,
+                         hipStream_t st);
 int soik_max_exponent(const double *x, int len, int nchunk, int *out, hipStream_t st);
 int soik_compress(int *out, long stride, const double *x, int len, int nchunk, int e_max,
                   const int *emi, int *nwords, const int *e_max_dev, hipStream_t st);
