@@ -645,22 +645,25 @@ __global__ void k_filter_mfma_table(const double *__restrict__ taps, unsigned sh
   }
 }
 
-// Blocks per transform of a complex128 MFMA filter launch.  One transform: 256 (one per CU, each
-// walking a contiguous range of tiles).  A batched launch (blockIdx.y = member) shares about two
-// rounds of blocks over all its members, so that each block's prologue (its B operands: up to
-// 160 KB of tap table at S = 16) is spent over many tiles also when the members are small.
+// Blocks per transform of a complex128 MFMA filter launch with per_cu blocks resident on a CU: as
+// many as the GPU holds at once, each walking a contiguous range of tiles.  (One block a CU left
+// the CUs at two or four waves for S = 4 and 8: N = 2^24 took 532 and 305 us.)  A batched launch
+// (blockIdx.y = member) shares about two rounds of blocks over all its members, so that each
+// block's prologue (its B operands: up to 160 KB of tap table at S = 16) is spent over many tiles
+// also when the members are small.
 // Every whole tile goes through the same loop body, so a member's results do not depend on how
 // its tiles are split over blocks (the complex64 kernels write each block's last tile through a
 // separate code copy and keep the single-transform split, so that batched results stay
-// bit-identical to eager ones).  SOI_FILTER_BATCH_BLOCKS sets the total (0: 256 per member).
-static long mfma_blocks_per_member(const SoiFilterArgs *a)
+// bit-identical to eager ones).  SOI_FILTER_BATCH_BLOCKS sets the total of a batch (0: as for one
+// transform).
+static long mfma_blocks_per_member(const SoiFilterArgs *a, long per_cu)
 {
   static const long total = [] {
     const char *e = getenv("SOI_FILTER_BATCH_BLOCKS");
-    return e ? atol(e) : 512L;
+    return e ? atol(e) : -1L;
   }();
-  if (a->b.n <= 1 || total <= 0) return 256;
-  const long nb = (total + a->b.n - 1) / a->b.n;
+  if (a->b.n <= 1 || total == 0) return 256 * per_cu;
+  const long nb = ((total > 0 ? total : 512 * per_cu) + a->b.n - 1) / a->b.n;
   return nb < 1 ? 1 : nb;
 }
 
@@ -1167,9 +1170,11 @@ template <int S, int LPW> struct Mfma64Cfg {
 };
 
 constexpr int mfma64_threads(int S, int LPW) { return S / LPW * 64; }
-
+// Waves a CU holds: 141 - 150 registers up to S = 16 (twelve waves: three blocks at S = 8, six at
+// S = 4; a block of S = 16 has eight, and a second one does not fit), all 256 at S = 32
+constexpr int mfma64_waves(int S) { return S <= 8 ? 12 : 8; }
 template <int S, int LPW>
-__global__ __launch_bounds__(mfma64_threads(S, LPW), mfma64_threads(S, LPW) / 256) void k_filter_mfma64(
+__global__ __launch_bounds__(mfma64_threads(S, LPW), mfma64_waves(S) / 4) void k_filter_mfma64(
     const double2 *__restrict__ x, double2 *__restrict__ at, const double *__restrict__ wt,
     const double2 *__restrict__ post, const double2 *__restrict__ twS, long M, long Mh, long nJ,
     int tiles_per_block, SoiBatch b)
@@ -1224,7 +1229,6 @@ __global__ __launch_bounds__(mfma64_threads(S, LPW), mfma64_threads(S, LPW) / 25
   const int am = n & 7, apart = n >> 3;
   const int v0 = (12 * am + g) * S + wave;
   int base = (int)((t0 * AC) % RC);  // ring slot of the tile's first chunk
-  const double *ringd = reinterpret_cast<const double *>(ring);
 
   // One tile.  PART: the transform's last tile when it holds fewer than TJ row groups (its
   // stores are predicated per row; it is never followed by another tile of this block).
@@ -1243,33 +1247,27 @@ __global__ __launch_bounds__(mfma64_threads(S, LPW), mfma64_threads(S, LPW) / 25
     const int ln = tv & 63, nv = ln & 15, gv = ln >> 4;
 
     // ---- MFMA: one accumulation chain per lane i, all on v_mfma_f64_16x16x4_f64
-    // A operand addresses.  For S >= 16 a K step advances by whole chunks (4S/64) and the lanes
-    // i of a wave stay inside one chunk, so a read is the lane's first address of the tile plus
-    // a compile-time offset, minus the ring length once the lane's chunk wraps.  (Per-read
-    // offsets computed once for the kernel would be loop-invariant and hoisted: 80 live
-    // registers.)  Smaller S take the chunk and offset of each read from its value index.
+    // A operand addresses.  NB K steps of 4S values make a whole number of chunks (one of S / 16
+    // at S >= 16, four or two a chunk below), and the lanes i of a wave stay inside one chunk, so a
+    // read is one of the lane's NB first addresses of the tile plus a compile-time offset, minus
+    // the ring length once its chunk wraps.  (Per-read offsets computed once for the kernel would
+    // be loop-invariant and hoisted: 40 - 80 live registers.)
     constexpr int CPB = CP * 16;            // chunk pitch in bytes
-    int a0 = 0, a0w = 0, wrap = 0;
-    if constexpr (S >= 16) {
-      int sb = base + (v0 >> 6);
+    constexpr int NB = 4 * S < CH ? CH / (4 * S) : 1, CS = 4 * S * NB / CH;
+    int a0[NB], wrap[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int v = v0 + 4 * j * S;
+      int sb = base + (v >> 6);
       if (sb >= RC) sb -= RC;
-      a0 = sb * CPB + (v0 & 63) * 16 + apart * 8;
-      a0w = a0 - RC * CPB;
-      wrap = RC - sb;
+      a0[j] = sb * CPB + (v & 63) * 16 + apart * 8;
+      wrap[j] = RC - sb;
     }
     const char *ringb = reinterpret_cast<const char *>(ring);
     auto aread = [&](int ks, int li) -> double {
-      if constexpr (S >= 16) {
-        constexpr int CS = 4 * S / 64;      // chunks per K step
-        const int cs = ks * CS;
-        const int ab = cs >= wrap ? a0w : a0;
-        return *reinterpret_cast<const double *>(ringb + ab + cs * CPB + li * NW * 16);
-      } else {
-        const int v = v0 + 4 * ks * S + li * NW;
-        int slot = base + (v >> 6);
-        if (slot >= RC) slot -= RC;
-        return ringd[2 * (slot * CP + (v & 63)) + apart];
-      }
+      const int j = ks % NB, cs = ks / NB * CS;
+      const int ab = cs >= wrap[j] ? a0[j] - RC * CPB : a0[j];
+      return *reinterpret_cast<const double *>(ringb + ab + cs * CPB + li * NW * 16);
     };
     // software pipeline: the A operands of step ks + 1 are read while step ks multiplies; the
     // scheduling barriers keep every read from being hoisted to the top of the block
@@ -1382,7 +1380,7 @@ template <int S, int LPW> static int launch_mfma64(const SoiFilterArgs *a, hipSt
   static_assert(CF::LDS_BYTES <= 160 * 1024, "complex128 MFMA filter exceeds LDS");
   if ((long)CF::RC * CF::CH > a->M * S) return (int)hipErrorInvalidValue;  // wraps at most once
   const long ntiles = (a->nJ + CF::TJ - 1) / CF::TJ;
-  long nb = mfma_blocks_per_member(a);
+  long nb = mfma_blocks_per_member(a, mfma64_waves(S) / CF::NWAVES);
   if (nb > ntiles) nb = ntiles;
   const int tpb = (int)((ntiles + nb - 1) / nb);
   nb = (ntiles + tpb - 1) / tpb;
@@ -1398,7 +1396,7 @@ static int filter_mfma64(const SoiFilterArgs *a, hipStream_t st)
   switch (a->S) {
     case 4: return launch_mfma64<4, 2>(a, st);
     case 8: return launch_mfma64<8, 2>(a, st);
-    case 16: return launch_mfma64<16, 2>(a, st);
+    case 16: return launch_mfma64<16, 4>(a, st);
     case 32: return launch_mfma64<32, 4>(a, st);
     default: return (int)hipErrorInvalidValue;
   }
