@@ -17,7 +17,8 @@ LIB = os.path.join(HERE, "libsoi_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = os.environ.get("SOI_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["soi_filter.hip", "soi_kernels.hip", "soi_fft.hip", "soi_fft_cols64.hip",
+HIP_SOURCES = ["soi_filter.hip", "soi_filter_g54.hip", "soi_filter_g87.hip",
+               "soi_filter_grt.hip", "soi_kernels.hip", "soi_fft.hip", "soi_fft_cols64.hip",
                "soi_fft_cols32.hip", "soi_fft_rows64.hip", "soi_fft_rows32.hip",
                "soi_fft_long32.hip"]
 C_SOURCES = ["pfft.c", "compress_host.c", "harness.c"]

@@ -197,6 +197,7 @@ static int plan_filter(soi_plan_t *pl, int window_mode)
             "16, 32 or 64)", pl->S, pl->n_mu, pl->d_mu, pl->B);
     return -1;
   }
+  a->taps_used = pl->B;
   a->M = pl->M;
   a->Mh = pl->Mh;
   a->nJ = pl->M / pl->d_mu;
@@ -206,6 +207,31 @@ static int plan_filter(soi_plan_t *pl, int window_mode)
     return -1;
   }
   return 0;
+}
+
+/* The lane-group MFMA filter (soi_filter_g.hpp) for the plan's taps: sets a->nk, the K steps that
+ * cover B + d (ND - 1) taps among those that have a kernel.  0 where it has none or where a tile's
+ * rows (at most 7 * 14 + 4 * 22, in whole chunks) would wrap more than once. */
+static int plan_filter_g(SoiFilterArgs *a)
+{
+  static const int k54[] = {10, 13, 16, 20, 22, 0}, k87[] = {16, 20, 22, 0}, krt[] = {20, 22, 0};
+  const int *k = a->n_mu == 8 ? k87 : a->ct ? k54 : krt;
+  const int need = a->taps_used + (a->n_mu == 8 ? 7 : 8);
+  if (a->M < 208) return 0;
+  while (*k && 4 * *k < need) ++k;
+  if (a->n_mu == 8 && *k == 22 && a->S > 16) return 0; /* does not fit LDS */
+  a->nk = *k;
+  return *k;
+}
+static size_t filter_g_table_bytes(const SoiFilterArgs *a)
+{
+  return (size_t)a->S * a->nk * 64 * sizeof(double) * (a->ct ? 2 : 1);
+}
+static int filter_g_table(const SoiFilterArgs *a, const double *taps, void *wt, hipStream_t st)
+{
+  return a->n_mu == 8 ? soik_filter_g87(a, 1, taps, wt, st)
+         : a->ct ? soik_filter_g54(a, 1, taps, wt, st)
+                 : soik_filter_grt(a, 1, taps, wt, st);
 }
 
 /* largest T in {8,4,2,1} with n*T <= cap and T | other */
@@ -517,11 +543,9 @@ void init_soi_descriptor(soi_desc_t *d, MPI_Comm comm, cfft_size_t k)
       /* The complex128 filter contraction on MFMA (v_mfma_f64_16x16x4_f64) where the shape
        * allows: the default.  SOI_FILTER_MFMA64=0 selects the VALU form. */
       const char *em = getenv("SOI_FILTER_MFMA64");
-      if ((!em || atoi(em) != 0) &&
-          soik_filter_mfma_supported((int)S, d->n_mu, d->d_mu, pl->fa.ct, B_pad, 3)) {
-        HIPCHK(hipMalloc(&pl->wt, soik_filter_mfma_table_bytes((int)S, B_pad, 3)));
-        KCHK(soik_filter_mfma_table((const double *)pl->taps, pl->wt, (int)S, B_pad, 3,
-                                    pl->stream));
+      if ((!em || atoi(em) != 0) && plan_filter_g(&pl->fa)) {
+        HIPCHK(hipMalloc(&pl->wt, filter_g_table_bytes(&pl->fa)));
+        KCHK(filter_g_table(&pl->fa, (const double *)pl->taps, pl->wt, pl->stream));
         pl->fa.wt = pl->wt;
         pl->fa.mfma = 3;
       }

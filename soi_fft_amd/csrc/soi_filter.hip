@@ -645,28 +645,6 @@ __global__ void k_filter_mfma_table(const double *__restrict__ taps, unsigned sh
   }
 }
 
-// Blocks per transform of a complex128 MFMA filter launch with per_cu blocks resident on a CU: as
-// many as the GPU holds at once, each walking a contiguous range of tiles.  (One block a CU left
-// the CUs at two or four waves for S = 4 and 8: N = 2^24 took 532 and 305 us.)  A batched launch
-// (blockIdx.y = member) shares about two rounds of blocks over all its members, so that each
-// block's prologue (its B operands: up to 160 KB of tap table at S = 16) is spent over many tiles
-// also when the members are small.
-// Every whole tile goes through the same loop body, so a member's results do not depend on how
-// its tiles are split over blocks (the complex64 kernels write each block's last tile through a
-// separate code copy and keep the single-transform split, so that batched results stay
-// bit-identical to eager ones).  SOI_FILTER_BATCH_BLOCKS sets the total of a batch (0: as for one
-// transform).
-static long mfma_blocks_per_member(const SoiFilterArgs *a, long per_cu)
-{
-  static const long total = [] {
-    const char *e = getenv("SOI_FILTER_BATCH_BLOCKS");
-    return e ? atol(e) : -1L;
-  }();
-  if (a->b.n <= 1 || total == 0) return 256 * per_cu;
-  const long nb = ((total > 0 ? total : 512 * per_cu) + a->b.n - 1) / a->b.n;
-  return nb < 1 ? 1 : nb;
-}
-
 template <int S> static int launch_mfma(const SoiFilterArgs *a, hipStream_t st)
 {
   typedef MfmaCfg<S> CF;
@@ -1108,299 +1086,7 @@ __global__ __launch_bounds__(mfma32_threads(S, LPW), mfma32_threads(S, LPW) / 25
   else run(std::false_type{});
 }
 
-// ---------------------------------------------------------------------------------------------
-// Complex128 real-tap filter on MFMA (v_mfma_f64_16x16x4_f64, FP64 products and accumulation).
-// The GEMM of each lane i is the one of the FP32 MFMA form with the rows ordered part-major,
-//   C[8 part + m][theta + 5D] = sum_k x_i[4 J0 + 12 m + k].part * t_i[theta][k - 4D],
-// m < 8, D < 3 (24 row groups J = J0 + 3m + D per tile), K = 80 >= BPAD + 8 in 20 four-deep
-// steps.  Lane layout (checked by soik_mfma64_layout_probe): A[row][k] in lane row + 16k,
-// B[k][col] in lane col + 16k, D[row][col] in lane col + 16 (row % 4), register row / 4.  With
-// part-major rows, lane col + 16g holds m = g (registers 0 and 2: real and imaginary part) and
-// m = 4 + g (registers 1 and 3).
-//
-// Wave w of the NW = S / LPW waves owns the lanes i = NW li + w, li < LPW.  The S-point DFT of
-// each output row R then splits as i = NW li + w, s = s1 + LPW s2:
-//   X[s] = sum_w w_NW^{w s2} [ w_S^{w s1} sum_li gamma[NW li + w] w_LPW^{li s1} ],
-// the LPW-point DFTs in the registers of the wave that holds the lanes, then one exchange
-// through LDS and an NW-point DFT per (R, s1), whose NW results go straight to HBM.
-//
-// A complex128 tile (164 input rows, 82 KB at S = 32) and its output rows (61 KB) do not fit
-// twice in LDS, so the input rows live in a ring of RC one-KB chunks (the direct-to-LDS load of
-// one wave, each followed by a 16-byte gap): the tile of row groups [24t, 24t + 24) reads chunks
-// [AC t, AC t + RC) of the input, slot = chunk mod RC, and the AC chunks that tile t + 1 adds
-// overwrite the AC slots that only tile t reads.  Those loads are issued as soon as tile t's
-// MFMA block is done and complete under its epilogue.  The B operands (taps, 20 per lane i)
-// stay in registers.
-// ---------------------------------------------------------------------------------------------
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2g __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) f64x2g gf64x2;
-
-// non-temporal store of one complex128 value through a global-address-space pointer: a flat
-// store would also count against LDS traffic, and the compiler then waits for the in-flight
-// direct-to-LDS loads before it
-__device__ __forceinline__ void store_nt_global(gf64x2 *p, double2 v)
-{
-  __builtin_nontemporal_store(f64x2g{v.x, v.y}, p);
-}
-
-template <int S, int LPW> struct Mfma64Cfg {
-  static constexpr int TJ = 24;                 // row groups per tile
-  static constexpr int NK = 20;                 // four-deep K steps
-  static constexpr int K = 4 * NK;
-  static constexpr int ROWS = 12 * 7 + K;       // input rows read per tile
-  static constexpr int ADV = TJ * 4;            // rows from one tile to the next
-  static constexpr int CH = 64;                 // complex128 values per wave-wide load (1 KB)
-  static constexpr int CP = CH + 1;             // chunk pitch in LDS: a 16-byte gap
-  static constexpr int RC = (ROWS * S + CH - 1) / CH;  // ring chunks: one tile's rows
-  static constexpr int AC = ADV * S / CH;       // chunks added per tile
-  static constexpr int NWAVES = S / LPW;
-  static constexpr int T = NWAVES * 64;
-  static constexpr int GR = TJ * 5;             // output rows R per tile
-  static constexpr int GP = S + 1;              // exchange row pitch: [R][s1 * NWAVES + w]
-  static constexpr int NTASK = GR * LPW;        // (R, s1) tasks of the cross-wave DFT
-  static constexpr int NC = (NTASK + T - 1) / T;
-  // DUP: the idle lanes of the last task slot repeat tasks of their own wave (every wave then
-  // issues the same NC * NWAVES stores per tile); otherwise whole waves would be idle
-  static constexpr int DUPD = NC * T - NTASK;
-  static constexpr bool DUP = DUPD < 64;
-  static_assert(ADV * S % CH == 0 && AC <= RC, "ring shape");
-  static_assert(LPW == 2 || LPW == 4 || LPW == 8, "in-register DFT size");
-  static constexpr int LDS_BYTES = (RC * CP + GR * GP + S + 5 * S) * 16;
-};
-
-constexpr int mfma64_threads(int S, int LPW) { return S / LPW * 64; }
-// Waves a CU holds: 141 - 150 registers up to S = 16 (twelve waves: three blocks at S = 8, six at
-// S = 4; a block of S = 16 has eight, and a second one does not fit), all 256 at S = 32
-constexpr int mfma64_waves(int S) { return S <= 8 ? 12 : 8; }
-template <int S, int LPW>
-__global__ __launch_bounds__(mfma64_threads(S, LPW), mfma64_waves(S) / 4) void k_filter_mfma64(
-    const double2 *__restrict__ x, double2 *__restrict__ at, const double *__restrict__ wt,
-    const double2 *__restrict__ post, const double2 *__restrict__ twS, long M, long Mh, long nJ,
-    int tiles_per_block, SoiBatch b)
-{
-  typedef Mfma64Cfg<S, LPW> CF;
-  x = batch_ptr(x, b.x);
-  at = batch_ptr(at, b.at);
-  constexpr int NK = CF::NK, CH = CF::CH, CP = CF::CP, RC = CF::RC, AC = CF::AC;
-  constexpr int NW = CF::NWAVES, GP = CF::GP;
-  gf64x2 *const atg = (gf64x2 *)at;
-  __shared__ __align__(16) double2 ring[RC * CP];
-  __shared__ __align__(16) double2 G[CF::GR * GP];
-  __shared__ __align__(16) double2 tw[S];
-  __shared__ __align__(16) double2 pfl[5 * S];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int n = lane & 15, g = lane >> 4;
-
-  double wb[LPW][NK];  // B operands of this wave's lanes i = NW li + wave
-#pragma unroll
-  for (int li = 0; li < LPW; ++li)
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) wb[li][ks] = wt[((li * NW + wave) * NK + ks) * 64 + lane];
-  for (int e = tid; e < S; e += CF::T) tw[e] = twS[e];
-  for (int e = tid; e < 5 * S; e += CF::T) pfl[e] = post[e];
-
-  const long ntiles = (nJ + CF::TJ - 1) / CF::TJ;
-  const long t0 = (long)blockIdx.x * tiles_per_block;
-  const long t1 = min(ntiles, t0 + tiles_per_block);
-  const long N = M * S;
-  if (t0 >= t1) return;
-
-  // input chunks [c0, c0 + cnt) into their ring slots (absolute chunk c -> slot c mod RC);
-  // a chunk is 64 consecutive values from element 64 c, wrapping at N
-  auto dma = [&](long c0, int cnt) {
-    int slot = (int)((c0 + wave) % RC);
-    for (int c = wave; c < cnt; c += NW) {
-      long gi = (c0 + c) * CH + lane;
-      if (gi >= N) gi -= N;
-      __builtin_amdgcn_global_load_lds((const void *)(x + gi), (lds_void_t *)(ring + slot * CP), 16,
-                                       0, 0);
-      slot += NW;
-      if (slot >= RC) slot -= RC;
-    }
-  };
-
-  dma(t0 * AC, RC);
-  wait_vmcnt<0>();
-  lds_barrier();
-
-  // A operand of lane (n, g): row (m, part) = (n & 7, n >> 3), k = g; value index within the
-  // tile (12 m + 4 ks + g) * S + i with i = NW li + wave
-  const int am = n & 7, apart = n >> 3;
-  const int v0 = (12 * am + g) * S + wave;
-  int base = (int)((t0 * AC) % RC);  // ring slot of the tile's first chunk
-
-  // One tile.  PART: the transform's last tile when it holds fewer than TJ row groups (its
-  // stores are predicated per row; it is never followed by another tile of this block).
-  // Whole tiles issue the same store instructions in every wave, unconditionally (in DUP
-  // mode idle lanes repeat a neighbour's task and store the same value to the same address),
-  // so that the compiler's wait tracking sees every one of them and the ring reads of the
-  // next tile wait only for the loads issued before them, not for the stores issued after.
-  auto body = [&](long tile, auto part_tag) {
-    constexpr bool PART = decltype(part_tag)::value;
-    const bool more = !PART && tile + 1 < t1;
-    // the epilogue's per-thread indices and addresses are recomputed each tile from an opaque
-    // copy of the thread index: hoisted out of the tile loop they would stay live through the
-    // MFMA block, beside the 20 B operands per lane i
-    int tv = tid;
-    asm volatile("" : "+v"(tv));
-    const int ln = tv & 63, nv = ln & 15, gv = ln >> 4;
-
-    // ---- MFMA: one accumulation chain per lane i, all on v_mfma_f64_16x16x4_f64
-    // A operand addresses.  NB K steps of 4S values make a whole number of chunks (one of S / 16
-    // at S >= 16, four or two a chunk below), and the lanes i of a wave stay inside one chunk, so a
-    // read is one of the lane's NB first addresses of the tile plus a compile-time offset, minus
-    // the ring length once its chunk wraps.  (Per-read offsets computed once for the kernel would
-    // be loop-invariant and hoisted: 40 - 80 live registers.)
-    constexpr int CPB = CP * 16;            // chunk pitch in bytes
-    constexpr int NB = 4 * S < CH ? CH / (4 * S) : 1, CS = 4 * S * NB / CH;
-    int a0[NB], wrap[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int v = v0 + 4 * j * S;
-      int sb = base + (v >> 6);
-      if (sb >= RC) sb -= RC;
-      a0[j] = sb * CPB + (v & 63) * 16 + apart * 8;
-      wrap[j] = RC - sb;
-    }
-    const char *ringb = reinterpret_cast<const char *>(ring);
-    auto aread = [&](int ks, int li) -> double {
-      const int j = ks % NB, cs = ks / NB * CS;
-      const int ab = cs >= wrap[j] ? a0[j] - RC * CPB : a0[j];
-      return *reinterpret_cast<const double *>(ringb + ab + cs * CPB + li * NW * 16);
-    };
-    // software pipeline: the A operands of step ks + 1 are read while step ks multiplies; the
-    // scheduling barriers keep every read from being hoisted to the top of the block
-    f64x4 acc[LPW];
-    double acur[LPW];
-#pragma unroll
-    for (int li = 0; li < LPW; ++li) {
-      acc[li] = f64x4{0, 0, 0, 0};
-      acur[li] = aread(0, li);
-    }
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      double anxt[LPW];
-      if (ks + 1 < NK) {
-#pragma unroll
-        for (int li = 0; li < LPW; ++li) anxt[li] = aread(ks + 1, li);
-      }
-#pragma unroll
-      for (int li = 0; li < LPW; ++li)
-        acc[li] = __builtin_amdgcn_mfma_f64_16x16x4f64(acur[li], wb[li][ks], acc[li], 0, 0, 0);
-      if (ks + 1 < NK) {
-#pragma unroll
-        for (int li = 0; li < LPW; ++li) acur[li] = anxt[li];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    lds_barrier();  // every wave is done reading this tile's rows and the previous tile's G
-    if (more) dma((tile + 1) * AC + RC - AC, AC);  // the next tile's new chunks, into dead slots
-    base += AC;
-    if (base >= RC) base -= RC;
-
-    // ---- post phase and the LPW-point DFTs over this wave's lanes i, twiddled by w_S^{w s1},
-    // into the exchange rows: G[R][s1 * NW + w].  Registers h and h + 2 are the real and
-    // imaginary part of row m = 4h + g; column nv = theta + 5D (15 is the unused column).
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      double2 v[LPW];
-#pragma unroll
-      for (int li = 0; li < LPW; ++li)
-        v[li] = cmul(double2{acc[li][h], acc[li][h + 2]}, pfl[(nv % 5) * S + li * NW + wave]);
-      dft_r<LPW>(v);
-      if (nv < 15) {
-        double2 *gr = G + (15 * (4 * h + gv) + nv) * GP + wave;
-        gr[0] = v[0];
-#pragma unroll
-        for (int s1 = 1; s1 < LPW; ++s1) gr[s1 * NW] = cmul(v[s1], tw[(wave * s1) % S]);
-      }
-    }
-    lds_barrier();
-
-    // ---- NW-point DFT over the waves for each (R, s1), stored segment-major: X[s1 + LPW s2]
-    // of row R = 5 J0 + r goes to alpha_tilde[s1 + LPW s2][R]; consecutive lanes take
-    // consecutive r, so each store instruction writes runs of consecutive R
-    const long R0 = tile * CF::TJ * 5;
-#pragma unroll
-    for (int c = 0; c < CF::NC; ++c) {
-      int e = tv + c * CF::T;
-      if constexpr (CF::DUP) {
-        if (e >= CF::NTASK) e -= CF::DUPD;
-      }
-      if (CF::DUP || CF::NTASK % CF::T == 0 || e < CF::NTASK) {
-        const int r = e % CF::GR, s1 = e / CF::GR;
-        double2 u[NW];
-#pragma unroll
-        for (int w = 0; w < NW; ++w) u[w] = G[r * GP + s1 * NW + w];
-        dft_r<NW>(u);
-        if (!PART || tile * CF::TJ + r / 5 < nJ) {
-#pragma unroll
-          for (int s2 = 0; s2 < NW; ++s2)
-            store_nt_global(atg + (long)(s1 + LPW * s2) * Mh + R0 + r, u[s2]);
-        }
-      }
-    }
-    // the next tile's chunks are complete once at most this wave's stores of this tile are
-    // outstanding (they were issued after the loads).  Unconditional on every path that loops
-    // back, so the compiler's wait tracking knows the ring is complete at the next tile.
-    if constexpr (!PART) {
-      asm volatile("" ::: "memory");
-      if constexpr (CF::DUP) wait_vmcnt<CF::NC * NW>();
-      else wait_vmcnt<0>();
-    }
-    lds_barrier();
-  };
-
-  // whole tiles in the loop; the transform's partial last tile, if this block has it, after it
-  const long tfull = min(t1, nJ / CF::TJ);
-  for (long tile = t0; tile < tfull; ++tile) body(tile, std::false_type{});
-  if (tfull < t1) body(tfull, std::true_type{});
-}
-
-// FP64 B operand table: wt[(i*NK + ks)*64 + lane] = t_i[theta][k - 4D] for k = 4 ks + lane/16
-// and col = lane % 16 = theta + 5D (zero for col 15 or a tap index outside [0, BPAD)), from the
-// FP64 real-tap table taps[(theta*S + i)*BPAD + b].
-__global__ void k_filter_mfma64_table(const double *__restrict__ taps, double *__restrict__ wt, int S,
-                                      int BPAD, int NK)
-{
-  const long total = (long)S * NK * 64;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
-    const int lane = (int)(e % 64), ks = (int)(e / 64 % NK), i = (int)(e / (64L * NK));
-    const int col = lane % 16, k = 4 * ks + lane / 16;
-    const int theta = col % 5, D = col / 5, bb = k - 4 * D;
-    const bool on = col < 15 && bb >= 0 && bb < BPAD;
-    wt[e] = on ? taps[((long)theta * S + i) * BPAD + bb] : 0.0;
-  }
-}
-
-template <int S, int LPW> static int launch_mfma64(const SoiFilterArgs *a, hipStream_t st)
-{
-  typedef Mfma64Cfg<S, LPW> CF;
-  static_assert(CF::LDS_BYTES <= 160 * 1024, "complex128 MFMA filter exceeds LDS");
-  if ((long)CF::RC * CF::CH > a->M * S) return (int)hipErrorInvalidValue;  // wraps at most once
-  const long ntiles = (a->nJ + CF::TJ - 1) / CF::TJ;
-  long nb = mfma_blocks_per_member(a, mfma64_waves(S) / CF::NWAVES);
-  if (nb > ntiles) nb = ntiles;
-  const int tpb = (int)((ntiles + nb - 1) / nb);
-  nb = (ntiles + tpb - 1) / tpb;
-  hipLaunchKernelGGL((k_filter_mfma64<S, LPW>), dim3((unsigned)nb, a->b.n > 0 ? a->b.n : 1),
-                     dim3(CF::T), 0, st, (const double2 *)a->x, (double2 *)a->at,
-                     (const double *)a->wt, (const double2 *)a->post, (const double2 *)a->twS, a->M,
-                     a->Mh, a->nJ, tpb, a->b);
-  return (int)hipGetLastError();
-}
-
-static int filter_mfma64(const SoiFilterArgs *a, hipStream_t st)
-{
-  switch (a->S) {
-    case 4: return launch_mfma64<4, 2>(a, st);
-    case 8: return launch_mfma64<8, 2>(a, st);
-    case 16: return launch_mfma64<16, 4>(a, st);
-    case 32: return launch_mfma64<32, 4>(a, st);
-    default: return (int)hipErrorInvalidValue;
-  }
-}
 
 // FP32 B operand table: wt[(i*NK + ks)*64 + lane] = t_i[theta][k - 4D] for k = 4 ks + lane/16
 // and n = lane % 16 = theta + 5D (zero for n = 15 or a tap index outside [0, BPAD)), rounded
@@ -1450,19 +1136,18 @@ static int filter_mfma32(const SoiFilterArgs *a, hipStream_t st)
   }
 }
 
-// The MFMA forms apply to the complex64 real-tap (5, 4) filter with S in {4, 8, 16, 32} and at
+// These MFMA forms apply to the complex64 real-tap (5, 4) filter with S in {4, 8, 16, 32} and at
 // most 88 (split-bf16, mode 1) or 72 (FP32, mode 2) padded taps.
 extern "C" int soik_filter_mfma_supported(int S, int n_mu, int d_mu, int ct, int BPAD, int mode)
 {
   const int maxb = mode == 1 ? 88 : Mfma32Cfg<4, 2>::K - 8;
-  return (mode == 1 || mode == 2 || mode == 3) && !ct && n_mu == 5 && d_mu == 4 && BPAD <= maxb &&
+  return (mode == 1 || mode == 2) && !ct && n_mu == 5 && d_mu == 4 && BPAD <= maxb &&
          (S == 4 || S == 8 || S == 16 || S == 32);
 }
 
 extern "C" size_t soik_filter_mfma_table_bytes(int S, int BPAD, int mode)
 {
   (void)BPAD;
-  if (mode == 3) return (size_t)S * Mfma64Cfg<4, 2>::NK * 64 * sizeof(double);
   if (mode == 2) return (size_t)S * Mfma32Cfg<4, 2>::NK * 64 * sizeof(float);
   return (size_t)S * MfmaCfg<4>::NCH * 3 * 64 * 16;
 }
@@ -1470,10 +1155,7 @@ extern "C" size_t soik_filter_mfma_table_bytes(int S, int BPAD, int mode)
 extern "C" int soik_filter_mfma_table(const double *taps, void *wt, int S, int BPAD, int mode,
                                       hipStream_t st)
 {
-  if (mode == 3)
-    hipLaunchKernelGGL(k_filter_mfma64_table, dim3(64), dim3(256), 0, st, taps, (double *)wt, S,
-                       BPAD, Mfma64Cfg<4, 2>::NK);
-  else if (mode == 2)
+  if (mode == 2)
     hipLaunchKernelGGL(k_filter_mfma32_table, dim3(64), dim3(256), 0, st, taps, (float *)wt, S,
                        BPAD, Mfma32Cfg<4, 2>::NK);
   else
@@ -1636,7 +1318,10 @@ extern "C" size_t soik_filter_lds_bytes(const SoiFilterArgs *a)
 
 extern "C" int soik_filter_sdft(const SoiFilterArgs *a, hipStream_t st)
 {
-  if (a->wt && a->mfma == 3 && !a->f32) return filter_mfma64(a, st);
+  if (a->wt && a->mfma == 3 && !a->f32)
+    return a->n_mu == 8 ? soik_filter_g87(a, 0, nullptr, nullptr, st)
+           : a->ct ? soik_filter_g54(a, 0, nullptr, nullptr, st)
+                   : soik_filter_grt(a, 0, nullptr, nullptr, st);
   if (a->f32 && a->wt) return a->mfma == 2 ? filter_mfma32(a, st) : filter_mfma(a, st);
   if (!a->ct) {
     RT_CASE(4, 32, 16) RT_CASE(4, 36, 16) RT_CASE(4, 40, 16)

@@ -38,7 +38,10 @@ typedef struct SoiFilterArgs {
   const void *wt;     /* tap operands of an MFMA form (NULL: VALU form) */
   long M, Mh, nJ;
   int S, n_mu, d_mu, BP, NP, NT, U, W, ct, f32;
-  int mfma;           /* MFMA form of wt: 1 = split-bf16 pieces, 2 = FP32, 3 = FP64 (complex128) */
+  int mfma;           /* MFMA form of wt: 1 = split-bf16 pieces, 2 = FP32, 3 = FP64 (complex128,
+                       * soi_filter_g.hpp) */
+  int taps_used;      /* B (taps beyond it are zero) */
+  int nk;             /* form 3: four-deep K steps */
   SoiBatch b;         /* batched launch tables (x -> b.x[t], at -> b.at[t]) */
 } SoiFilterArgs;
 
@@ -54,6 +57,9 @@ int soik_filter_mfma_supported(int S, int n_mu, int d_mu, int ct, int BPAD, int 
 size_t soik_filter_mfma_table_bytes(int S, int BPAD, int mode);
 int soik_filter_mfma_table(const double *taps, void *wt, int S, int BPAD, int mode,
                            hipStream_t st);
+int soik_filter_g54(const SoiFilterArgs *a, int kind, const double *taps, void *wt, hipStream_t st);
+int soik_filter_g87(const SoiFilterArgs *a, int kind, const double *taps, void *wt, hipStream_t st);
+int soik_filter_grt(const SoiFilterArgs *a, int kind, const double *taps, void *wt, hipStream_t st);
 int soik_fft_single(const soi_c64_t *at, soi_c64_t *X, const soi_c64_t *tw,
                     const soi_c64_t *winv, long L, long M, int S, int count, SoiBatch b, hipStream_t st);
 int soik_fft_col(soi_c64_t *data, const soi_c64_t *tw1, const soi_c64_t *thi,
