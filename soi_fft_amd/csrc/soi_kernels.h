@@ -109,11 +109,14 @@ int soik_compress(int *out, long stride, const double *x, int len, int nchunk, i
                   const int *emi, int *nwords, const int *e_max_dev, hipStream_t st);
 int soik_decompress(double *out, const int *in, long stride, int len, int nchunk, int e_max,
                     const int *emi, const int *e_max_dev, hipStream_t st);
-/* VLC planning on the device: out = [total, seg_max[S], send_counts[S], boundaries[P+1]] */
+/* VLC planning on the device: out = [total, seg_max[S], send_counts[S], boundaries[P+1]]; unused
+ * arguments are ignored */
 int soik_vlc_plan(const int *exps, int S, int P, int k, long l, long Mh, double ratio, int *emi,
-                  int *out, double *pcs, long *upre, int *nwords, hipStream_t st);
+                  int *out, double *pcs, long *unused, int *nwords, hipStream_t st);
+int soik_vlc_exchange(int *out, long stride, double *x, int len, int nchunk, const int *e_max_dev,
+                      const int *emi, hipStream_t st);
 int soik_compress_flat(int *out, long stride, const double *x, int len, int nchunk,
-                       const int *e_max_dev, const int *emi, const long *upre, hipStream_t st);
+                       const int *e_max_dev, const int *emi, const long *unused, hipStream_t st);
 int soik_decompress_flat(double *out, const int *in, long stride, int len, int nchunk,
                          const int *e_max_dev, const int *emi, hipStream_t st);
 int soik_gen_uniform(soi_c64_t *x, long N, uint64_t seed, hipStream_t st);

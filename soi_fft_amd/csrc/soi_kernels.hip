@@ -280,10 +280,9 @@ __device__ __forceinline__ VlcParams vlc_params(int e_max, int e_max_i)
   return v;
 }
 
-// The bit pattern of one element: i1Len bits of i1 (when i1Len > 0) followed by i2Len bits of
-// i2, as a value of fbits <= 56 bits, MSB first.  vec=1: rint + fmsub (compress.c:230-280);
-// vec=0: round() + unfused (compress.c:333-342).
-__device__ __forceinline__ uint64_t vlc_encode(double x, const VlcParams &v, bool vec)
+// The two integers of one element, i1 and i2 (their low i1Len and i2Len bits are sent).
+// vec=1: rint + fmsub (compress.c:230-280); vec=0: round() + unfused (compress.c:333-342).
+__device__ __forceinline__ uint2 vlc_ints(double x, const VlcParams &v, bool vec)
 {
   double d1, d2;
   if (vec) {
@@ -294,10 +293,17 @@ __device__ __forceinline__ uint64_t vlc_encode(double x, const VlcParams &v, boo
     double pr = __dmul_rn(x, v.e2);
     d2 = round(__dsub_rn(pr, __dmul_rn(d1, v.e3)));
   }
-  uint32_t i1 = (uint32_t)(int32_t)d1, i2 = (uint32_t)(int32_t)d2;
-  uint64_t f2 = v.i2Len >= 32 ? (uint64_t)i2 : ((uint64_t)i2 & ((1ull << v.i2Len) - 1));
+  return uint2{(uint32_t)(int32_t)d1, (uint32_t)(int32_t)d2};
+}
+
+// The bit pattern of one element: i1Len bits of i1 (when i1Len > 0) followed by i2Len bits of
+// i2, as a value of fbits <= 56 bits, MSB first.
+__device__ __forceinline__ uint64_t vlc_encode(double x, const VlcParams &v, bool vec)
+{
+  const uint2 i = vlc_ints(x, v, vec);
+  uint64_t f2 = v.i2Len >= 32 ? (uint64_t)i.y : ((uint64_t)i.y & ((1ull << v.i2Len) - 1));
   if (v.i1Len > 0) {
-    uint64_t f1 = (uint64_t)i1 & ((1ull << v.i1Len) - 1);
+    uint64_t f1 = (uint64_t)i.x & ((1ull << v.i1Len) - 1);
     return (f1 << v.i2Len) | f2;
   }
   return f2;
@@ -357,50 +363,6 @@ __device__ __forceinline__ long compress_words(int len, const VlcParams &v)
   return (nvf * v.fbits + 31) / 32 * 16 + ((len - nvf * 16) * v.fbits + 31) / 32;
 }
 
-// Work units of the flat compress: one unit per run of VLC_RUN vector rows of one lane, then one
-// per tail word
-constexpr int VLC_RUN = 8;
-__device__ __forceinline__ long compress_units(int len, const VlcParams &v)
-{
-  if (v.i2Len <= 0) return 0;
-  const long nvf = len / 16;
-  const long vrows = (nvf * v.fbits + 31) / 32;
-  return (vrows + VLC_RUN - 1) / VLC_RUN * 16 + ((len - nvf * 16) * v.fbits + 31) / 32;
-}
-
-// Rows r0 <= r < r1 of lane `lane`'s vector stream (word r*16 + lane), packed in one pass: the
-// fields overlapping the rows are encoded once each and shifted in MSB first; fields past the
-// lane's nvf are zero padding.  Same words as compress_word.
-__device__ __forceinline__ void compress_run(const double *__restrict__ in, int *__restrict__ o,
-                                             long nvf, const VlcParams &v, long r0, long r1,
-                                             int lane)
-{
-  const int fbits = v.fbits;
-  const long pos = r0 * 32;
-  long f = (pos <= (long)UINT32_MAX) ? (long)((uint32_t)pos / (uint32_t)fbits) : pos / fbits;
-  int nb = fbits - (int)(pos - f * fbits);  // bits of field f at or after pos
-  uint64_t acc = 0;
-  int nacc = 0;
-  long r = r0;
-  while (r < r1) {
-    const uint64_t val = f < nvf ? vlc_encode(in[f * 16 + lane], v, true) : 0;
-    while (nb > 0 && r < r1) {
-      const int take = min(nb, 32 - nacc);
-      acc = (acc << take) | ((val >> (nb - take)) & ((1ull << take) - 1));
-      nacc += take;
-      nb -= take;
-      if (nacc == 32) {
-        o[r * 16 + lane] = (int)(uint32_t)acc;
-        ++r;
-        acc = 0;
-        nacc = 0;
-      }
-    }
-    ++f;
-    nb = fbits;
-  }
-}
-
 // compress: one thread per output word, blockIdx.y = chunk.  nwords[c] = compress()'s return
 // value.
 __global__ void k_compress(int *__restrict__ out, long stride, const double *__restrict__ x,
@@ -417,54 +379,6 @@ __global__ void k_compress(int *__restrict__ out, long stride, const double *__r
   for (long wi = blockIdx.x * (long)blockDim.x + threadIdx.x; wi < total;
        wi += (long)gridDim.x * blockDim.x)
     o[wi] = (int)compress_word(in, len, v, wi);
-}
-
-// compress over all chunks as one range of work units (upre: exclusive prefix of the chunks'
-// unit counts, nchunk + 1 entries, from k_vlc_plan): every block has the same share of units, a
-// contiguous span, whatever the chunks' field widths.  A thread finds the chunk of its first unit
-// by bisection and then walks forward: chunks hold thousands of units, so the walk rarely moves.
-__global__ void k_compress_flat(int *__restrict__ out, long stride, const double *__restrict__ x,
-                                int len, int nchunk, const int *__restrict__ e_max_dev,
-                                const int *__restrict__ emi, const long *__restrict__ upre)
-{
-  const long total = upre[nchunk];
-  const long span = (total + gridDim.x - 1) / gridDim.x;
-  const long u1 = min(total, (blockIdx.x + 1) * span);
-  long u = blockIdx.x * span + threadIdx.x;
-  if (u >= u1) return;
-  int c = 0, hi = nchunk - 1;  // the last chunk c with upre[c] <= u: the one holding unit u
-  while (c < hi) {
-    const int mid = (c + hi + 1) >> 1;
-    if (upre[mid] <= u) c = mid;
-    else hi = mid - 1;
-  }
-  const int e_max = *e_max_dev;
-  const long nvf = len / 16;
-  long first = upre[c], next = upre[c + 1];
-  VlcParams v = vlc_params(e_max, emi[c]);
-  long vrows = (nvf * v.fbits + 31) / 32, nvu = (vrows + VLC_RUN - 1) / VLC_RUN * 16;
-  for (; u < u1; u += blockDim.x) {
-    if (next <= u) {
-      do {
-        ++c;
-        next = upre[c + 1];
-      } while (next <= u);
-      first = upre[c];
-      v = vlc_params(e_max, emi[c]);
-      vrows = (nvf * v.fbits + 31) / 32;
-      nvu = (vrows + VLC_RUN - 1) / VLC_RUN * 16;
-    }
-    const long q = u - first;
-    const double *in = x + (long)c * len;
-    int *o = out + (long)c * stride;
-    if (q < nvu) {
-      const long r0 = (q >> 4) * VLC_RUN;
-      compress_run(in, o, nvf, v, r0, min(vrows, r0 + VLC_RUN), (int)(q & 15));
-    } else {
-      const long wi = vrows * 16 + (q - nvu);
-      o[wi] = (int)compress_word(in, len, v, wi);
-    }
-  }
 }
 
 // extract the fbits-wide field f of a lane stream whose word w is at base[w*wstride]
@@ -487,6 +401,13 @@ __device__ __forceinline__ uint64_t vlc_field(const int *base, long wstride, lon
   return (bits >> sh) & ((fbits >= 64) ? ~0ull : ((1ull << fbits) - 1));
 }
 
+// the element that the two (sign-extended) integers stand for
+__device__ __forceinline__ double vlc_value(int32_t i1, int32_t i2, const VlcParams &v, bool vec)
+{
+  if (vec) return fma((double)i1, v.d1, (double)i2 * v.d2);       // compress.c:472-483
+  return __dadd_rn(__dmul_rn((double)i1, v.d1), __dmul_rn((double)i2, v.d2));  // :529-531
+}
+
 __device__ __forceinline__ double vlc_decode(uint64_t fv, const VlcParams &v, bool vec)
 {
   int32_t i1 = 0, i2;
@@ -497,8 +418,7 @@ __device__ __forceinline__ double vlc_decode(uint64_t fv, const VlcParams &v, bo
     uint64_t f1 = (fv >> v.i2Len) & ((1ull << v.i1Len) - 1);
     i1 = (int32_t)((int64_t)(f1 << (64 - v.i1Len)) >> (64 - v.i1Len));
   }
-  if (vec) return fma((double)i1, v.d1, (double)i2 * v.d2);       // compress.c:472-483
-  return __dadd_rn(__dmul_rn((double)i1, v.d1), __dmul_rn((double)i2, v.d2));  // :529-531
+  return vlc_value(i1, i2, v, vec);
 }
 
 // Element e of a chunk decoded from its stream w (compress.c:428-544)
@@ -527,29 +447,120 @@ __global__ void k_decompress(double *__restrict__ out, const int *__restrict__ i
     o[e] = decompress_elem(w, len, v, e);
 }
 
-// decompress over all chunks as one range of elements, a contiguous span per block
-__global__ void k_decompress_flat(double *__restrict__ out, const int *__restrict__ in,
-                                  long stride, int len, int nchunk,
-                                  const int *__restrict__ e_max_dev, const int *__restrict__ emi)
-{
-  const long total = (long)nchunk * len;
-  const long span = (total + gridDim.x - 1) / gridDim.x;
-  const long g1 = min(total, (blockIdx.x + 1) * span);
-  long g = blockIdx.x * span + threadIdx.x;
-  if (g >= g1) return;
-  const int e_max = *e_max_dev;
-  int c = (int)(g / len);
-  long e = g - (long)c * len;
-  VlcParams v = vlc_params(e_max, emi[c]);
-  for (; g < g1; g += blockDim.x, e += blockDim.x) {
-    if (e >= len) {
-      do {
-        e -= len;
-        ++c;
-      } while (e >= len);
-      v = vlc_params(e_max, emi[c]);
+// ---------------------------------------------------------------------------------------------
+// The exchange of one device: compress every chunk and (DECODE) decode it in place, in one pass.
+// 32 consecutive fields of a lane fill exactly fbits words, so a thread takes 32 fields of one
+// lane: no field is in two threads' words, each is encoded once, and its decoded value goes back over
+// the element that it came from.  All threads have the same work whatever the chunks' field
+// widths, and the 16 lanes of a vector row are adjacent threads (128-byte runs of elements, 64-byte
+// runs of words).  The scalar tail of a chunk (fewer than 16 elements) is one thread's.
+// Bound by memory: elements read once, words and elements written once.  N = 7*2^23 (1.07 GB of
+// elements, about 0.7 GB of words): 609 us, 4.7 TB/s; compressing and decompressing in two passes
+// over runs of words took 690 + 541 us.
+// ---------------------------------------------------------------------------------------------
+constexpr int VLC_FIELDS = 32;
+
+// One lane's bit stream, MSB first: word r goes to o[r * pitch]; cur holds the last nacc (< 32)
+// bits that are not in a word yet, below anything.  A field comes left-aligned, so that the
+// bits above it fall out of the shifts; the widths are the same in all lanes of a wave.
+struct VlcPack {
+  int *o;
+  int pitch;
+  uint32_t cur;
+  int nacc;
+  __device__ __forceinline__ void put(uint32_t left, int n)  // 1 <= n <= 32
+  {
+    if (nacc + n >= 32) {
+      *o = (int)__builtin_amdgcn_alignbit(cur, left, (uint32_t)nacc);
+      o += pitch;
+      nacc -= 32;
     }
-    out[g] = decompress_elem(in + (long)c * stride, len, v, e);
+    cur = __builtin_amdgcn_alignbit(cur, left, (uint32_t)(32 - n));
+    nacc += n;
+  }
+  __device__ __forceinline__ void flush()
+  {
+    if (nacc > 0) *o = (int)(cur << (32 - nacc));
+  }
+};
+
+// One element into the stream; returns the value that decoding it gives
+__device__ __forceinline__ double vlc_put(double x, const VlcParams &v, bool vec, VlcPack &w)
+{
+  const uint2 i = vlc_ints(x, v, vec);
+  int32_t i1 = 0;
+  if (v.i1Len > 0) {
+    const uint32_t left = i.x << (32 - v.i1Len);
+    w.put(left, v.i1Len);
+    i1 = (int32_t)left >> (32 - v.i1Len);
+  }
+  const uint32_t left = i.y << (32 - v.i2Len);
+  w.put(left, v.i2Len);
+  return vlc_value(i1, (int32_t)left >> (32 - v.i2Len), v, vec);
+}
+
+template <bool DECODE>
+__global__ __launch_bounds__(256) void k_vlc_exchange(int *__restrict__ out, long stride,
+                                                      double *__restrict__ x, int len, int nchunk,
+                                                      const int *__restrict__ e_max_dev,
+                                                      const int *__restrict__ emi)
+{
+  const int nvf = len / 16, ntail = len - nvf * 16;
+  const int nu = (nvf + VLC_FIELDS - 1) / VLC_FIELDS;
+  // a wave takes 4 neighbouring units of one chunk: the chunk and its widths are scalars
+  const int per = (nu + 3) / 4 + (ntail ? 1 : 0);
+  const long wv = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int c = (int)(wv / per), g = (int)(wv - (long)c * per);
+  if (c >= nchunk) return;
+  const int lane = threadIdx.x & 15, u = g * 4 + (((int)threadIdx.x >> 4) & 3);
+  const VlcParams v = vlc_params(*e_max_dev, emi[c]);
+  const bool coded = v.i2Len > 0;
+  double *xc = x + (long)c * len;
+  int *oc = out + (long)c * stride;
+  constexpr int G = 8;  // fields loaded together
+  if ((g + 1) * 4 * VLC_FIELDS <= nvf) {
+    double *p = xc + (long)u * (VLC_FIELDS * 16) + lane;
+    if (coded) {
+      VlcPack w = {oc + ((long)u * v.fbits) * 16 + lane, 16, 0, 0};
+      double a[G], b[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) a[i] = p[i * 16];
+#pragma unroll
+      for (int f = 0; f < VLC_FIELDS; f += G) {
+#pragma unroll
+        for (int i = 0; i < G; ++i) b[i] = a[i];
+        if (f + G < VLC_FIELDS) {
+#pragma unroll
+          for (int i = 0; i < G; ++i) a[i] = p[(f + G + i) * 16];
+        }
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          const double y = vlc_put(b[i], v, true, w);
+          if constexpr (DECODE) p[(f + i) * 16] = y;
+        }
+      }
+    } else if constexpr (DECODE) {
+#pragma unroll
+      for (int f = 0; f < VLC_FIELDS; ++f) p[f * 16] = 0.0;
+    }
+  } else if (g * 4 < nu) {  // the last units of the chunk
+    if (u >= nu) return;
+    double *p = xc + (long)u * (VLC_FIELDS * 16) + lane;
+    VlcPack w = {oc + ((long)u * v.fbits) * 16 + lane, 16, 0, 0};
+    const int nf = min(VLC_FIELDS, nvf - u * VLC_FIELDS);
+    for (int f = 0; f < nf; ++f) {
+      const double y = coded ? vlc_put(p[f * 16], v, true, w) : 0.0;
+      if constexpr (DECODE) p[f * 16] = y;
+    }
+    w.flush();
+  } else if ((threadIdx.x & 63) == 0) {  // the scalar tail
+    double *p = xc + (long)nvf * 16;
+    VlcPack w = {oc + ((long)nvf * v.fbits + 31) / 32 * 16, 1, 0, 0};
+    for (int f = 0; f < ntail; ++f) {
+      const double y = coded ? vlc_put(p[f], v, false, w) : 0.0;
+      if constexpr (DECODE) p[f] = y;
+    }
+    w.flush();
   }
 }
 
@@ -756,123 +767,145 @@ extern "C" int soik_decompress(double *out, const int *in, long stride, int len,
 // VLC planning on the device (pfft.c:316-343, 390-440): from the per-chunk exponents of the
 // S x P chunks (chunk (s, p) = s*P + p), the per-segment maximum (the reference's
 // MPI_Allreduce(MAX) over ranks), the global maximum, every chunk's segment exponent, the
-// per-segment send counts in doubles and the cost-balanced segment boundaries.  One block; the
-// boundary walk is sequential in thread 0 with the reference's double arithmetic, unfused, so
-// the boundaries are bit-identical to the host restatement.
+// per-segment send counts in doubles and the cost-balanced segment boundaries.  One block; only
+// the prefix sum of the costs is serial (the reference's double arithmetic, unfused and in its
+// order, so that the boundaries are bit-identical to the host restatement); its terms and the
+// boundary searches run on all threads (S = P = 64: 13 us, 56 us with the walk
+// and the terms serial).
 // out: [0] global maximum, [1 .. S] segment maxima, [1+S .. 2S] send counts,
 //      [1+2S .. 1+2S+P] segment boundaries; pcs: S + 1 doubles of scratch.
 __global__ void k_vlc_plan(const int *__restrict__ exps, int S, int P, int k, long l, long Mh,
                            double ratio, int *__restrict__ emi, int *__restrict__ out,
-                           double *__restrict__ pcs_g, long *__restrict__ upre,
-                           int *__restrict__ nwords)
+                           double *__restrict__ pcs_g, int *__restrict__ nwords)
 {
 #pragma clang fp contract(off)
-  // segment maxima and prefix costs in LDS when S is small enough (the serial walk below then
+  // segment maxima and prefix costs in LDS when S is small enough (the serial sum below then
   // reads no global memory), else in the caller's scratch
   constexpr int SMAX = 2048;
   __shared__ int smax, segs[SMAX];
   __shared__ double pcs_s[SMAX + 1];
   const bool inl = S <= SMAX;
   double *pcs = inl ? pcs_s : pcs_g;
-  if (threadIdx.x == 0) smax = INT_MIN;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  if (tid == 0) smax = INT_MIN;
+  if (inl)
+    for (int s = tid; s < S; s += nt) segs[s] = INT_MIN;
   __syncthreads();
-  for (int s = threadIdx.x; s < S; s += blockDim.x) {
-    int m = INT_MIN;
-    for (int p = 0; p < P; ++p) m = max(m, exps[s * P + p]);
-    out[1 + s] = m;
-    if (inl) segs[s] = m;
-    atomicMax(&smax, m);
+  if (inl) {
+    // the chunks of a segment over the threads: consecutive threads on consecutive chunks
+    for (int c = tid; c < S * P; c += nt) atomicMax(&segs[c / P], exps[c]);
+    __syncthreads();
+    for (int s = tid; s < S; s += nt) {
+      out[1 + s] = segs[s];
+      atomicMax(&smax, segs[s]);
+    }
+  } else {
+    for (int s = tid; s < S; s += nt) {
+      int m = INT_MIN;
+      for (int p = 0; p < P; ++p) m = max(m, exps[s * P + p]);
+      out[1 + s] = m;
+      atomicMax(&smax, m);
+    }
   }
   __syncthreads();
   const int total = smax;
-  for (int c = threadIdx.x; c < S * P; c += blockDim.x) emi[c] = inl ? segs[c / P] : out[1 + c / P];
-  if (upre) {
-    // work units per chunk (all chunks of a segment alike) and their exclusive prefix over the
-    // chunks, for k_compress_flat; nwords = compress()'s return value per chunk
-    const int len = (int)(2 * l);
-    __shared__ long useg_total;
-    if (threadIdx.x == 0) {
-      long acc = 0;
-      for (int s = 0; s < S; ++s) {
-        if (inl) pcs_s[s] = (double)acc;  // reused below as each segment's first unit (exact)
-        acc += compress_units(len, vlc_params(total, inl ? segs[s] : out[1 + s])) * P;
-      }
-      useg_total = acc;
-    }
-    __syncthreads();
-    for (int c = threadIdx.x; c < S * P; c += blockDim.x) {
-      const int s = c / P, p = c % P;
-      const VlcParams v = vlc_params(total, inl ? segs[s] : out[1 + s]);
-      long first = 0;
-      if (inl) {
-        first = (long)pcs_s[s];
-      } else {
-        for (int q = 0; q < s; ++q)
-          first += compress_units(len, vlc_params(total, out[1 + q])) * P;
-      }
-      upre[c] = first + compress_units(len, v) * p;
-      nwords[c] = (int)compress_words(len, v);
-    }
-    if (threadIdx.x == 0) upre[S * P] = useg_total;
-    __syncthreads();
+  // per segment: send count and cost (the term that the prefix sum adds), then per chunk
+  for (int s = tid; s < S; s += nt) {
+    int bits = 52 + 3 - (total - (inl ? segs[s] : out[1 + s]));
+    if (bits > 31) ++bits;
+    const int lenPerSimdLane = (int)((l * 2 / 16 * bits + 31) / 32);
+    const int remainder = (int)((l * 2 % 16 * bits + 31) / 32);
+    int sendLen = lenPerSimdLane * 16 + remainder;
+    if (bits <= 0) sendLen = 0;
+    const int cnt = (sendLen + 1) / 2;
+    out[1 + S + s] = cnt;
+    pcs[s + 1] = ratio * cnt / 2 / Mh;
   }
-  if (threadIdx.x != 0) return;
-  out[0] = total;
-  pcs[0] = 0;
-  for (int p = 0; p < P; ++p)
-    for (int ik = 0; ik < k; ++ik) {
-      const int s = p * k + ik;
-      int bits = 52 + 3 - (total - (inl ? segs[s] : out[1 + s]));
-      if (bits > 31) ++bits;
-      const int lenPerSimdLane = (int)((l * 2 / 16 * bits + 31) / 32);
-      const int remainder = (int)((l * 2 % 16 * bits + 31) / 32);
-      int sendLen = lenPerSimdLane * 16 + remainder;
-      if (bits <= 0) sendLen = 0;
-      const int cnt = (sendLen + 1) / 2;
-      out[1 + S + s] = cnt;
-      pcs[s + 1] = pcs[s] + ratio * cnt / 2 / Mh + 1;
+  const int len = (int)(2 * l);
+  for (int c = tid; c < S * P; c += nt) {
+    const int seg = inl ? segs[c / P] : out[1 + c / P];
+    emi[c] = seg;
+    nwords[c] = (int)compress_words(len, vlc_params(total, seg));
+  }
+  __syncthreads();
+  if (tid == 0) {
+    out[0] = total;
+    double acc = 0;
+    pcs[0] = 0;
+    for (int s = 0; s < S; ++s) {
+      acc = acc + pcs[s + 1] + 1;
+      pcs[s + 1] = acc;
     }
+  }
+  __syncthreads();
   int *bd = out + 1 + 2 * S;
-  bd[0] = 0;
-  bd[P] = S;
   const double costPerRank = pcs[S] / P;
-  int s = 1;
-  for (int p = 1; p < P;) {
-    const double target = p * costPerRank;
-    if (pcs[s] >= target) {
-      bd[p] = (pcs[s] - target > target - pcs[s - 1]) ? s - 1 : s;
-      ++p;
-    } else {
-      ++s;
+  if (tid == 0) bd[0] = 0, bd[P] = S;
+  if (ratio >= 0) {
+    // increasing costs: every boundary by itself, the first s >= 1 with pcs[s] >= target
+    for (int p = 1 + tid; p < P; p += nt) {
+      const double target = p * costPerRank;
+      int lo = 1, hi = S;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (pcs[mid] >= target) hi = mid;
+        else lo = mid + 1;
+      }
+      bd[p] = (pcs[lo] - target > target - pcs[lo - 1]) ? lo - 1 : lo;
+    }
+  } else if (tid == 0) {  // the reference's walk
+    int s = 1;
+    for (int p = 1; p < P;) {
+      const double target = p * costPerRank;
+      if (pcs[s] >= target) {
+        bd[p] = (pcs[s] - target > target - pcs[s - 1]) ? s - 1 : s;
+        ++p;
+      } else {
+        ++s;
+      }
     }
   }
 }
 
 extern "C" int soik_vlc_plan(const int *exps, int S, int P, int k, long l, long Mh, double ratio,
-                             int *emi, int *out, double *pcs, long *upre, int *nwords,
-                             hipStream_t st)
+                             int *emi, int *out, double *pcs, long *, int *nwords, hipStream_t st)
 {
-  hipLaunchKernelGGL(k_vlc_plan, dim3(1), dim3(256), 0, st, exps, S, P, k, l, Mh, ratio, emi, out,
-                     pcs, upre, nwords);
+  hipLaunchKernelGGL(k_vlc_plan, dim3(1), dim3(1024), 0, st, exps, S, P, k, l, Mh, ratio, emi, out,
+                     pcs, nwords);
   return (int)hipGetLastError();
 }
 
-// Flat compress / decompress of the nchunk chunks of one VLC exchange (after soik_vlc_plan)
+template <bool DECODE>
+static int vlc_exchange(int *out, long stride, double *x, int len, int nchunk, const int *e_max_dev,
+                        const int *emi, hipStream_t st)
+{
+  if (nchunk <= 0 || len <= 0) return 0;
+  const int nvf = len / 16, nu = (nvf + VLC_FIELDS - 1) / VLC_FIELDS;
+  const long waves = (long)nchunk * ((nu + 3) / 4 + (len % 16 ? 1 : 0));
+  hipLaunchKernelGGL(k_vlc_exchange<DECODE>, dim3(nblk(waves, 4)), dim3(256), 0, st, out, stride,
+                     x, len, nchunk, e_max_dev, emi);
+  return (int)hipGetLastError();
+}
+
+// Words of all chunks, and the chunks decoded from them in place (after soik_vlc_plan)
+extern "C" int soik_vlc_exchange(int *out, long stride, double *x, int len, int nchunk,
+                                 const int *e_max_dev, const int *emi, hipStream_t st)
+{
+  return vlc_exchange<true>(out, stride, x, len, nchunk, e_max_dev, emi, st);
+}
+
+// The two halves by themselves: the words (x stays), and decoding them
 extern "C" int soik_compress_flat(int *out, long stride, const double *x, int len, int nchunk,
-                                  const int *e_max_dev, const int *emi, const long *upre,
+                                  const int *e_max_dev, const int *emi, const long *,
                                   hipStream_t st)
 {
-  hipLaunchKernelGGL(k_compress_flat, dim3(2048), dim3(256), 0, st, out, stride, x, len, nchunk,
-                     e_max_dev, emi, upre);
-  return (int)hipGetLastError();
+  return vlc_exchange<false>(out, stride, const_cast<double *>(x), len, nchunk, e_max_dev, emi, st);
 }
 
 extern "C" int soik_decompress_flat(double *out, const int *in, long stride, int len, int nchunk,
                                     const int *e_max_dev, const int *emi, hipStream_t st)
 {
-  hipLaunchKernelGGL(k_decompress_flat, dim3(2048), dim3(256), 0, st, out, in, stride, len,
-                     nchunk, e_max_dev, emi);
-  return (int)hipGetLastError();
+  return soik_decompress(out, in, stride, len, nchunk, 0, emi, e_max_dev, st);
 }
 
 extern "C" int soik_gen_uniform(double2 *x, long N, uint64_t seed, hipStream_t st)
