@@ -94,6 +94,7 @@ typedef struct {
   /* fft */
   int fft_one;                     /* one pass, one segment per block (fft_single then too) */
   int fft_long;                    /* complex64 of N >= 2^24: the passes of soi_fft_long32.hip */
+  int fft_longd;                   /* ... of soi_fft_long32d.hip */
   int fft_single, single_count, fft_reg;
   int n1, n2, Tc, Tr, B1, lb1;
   int cvar, rvar;                  /* tile alternatives of the column and row pass in use */
@@ -348,6 +349,11 @@ static int plan_fft(soi_plan_t *pl)
   while ((long)b1 * b1 < Mh) b1 <<= 1, ++lb;
   pl->B1 = b1;
   pl->lb1 = lb;
+  if (pl->fft_long && soik_fft_longd_supported(bn1, 0) &&
+      soik_fft_longd_supported(bn2, 1)) {
+    pl->fft_longd = pl->fft_reg = 1;
+    pl->Mt = (long)(pl->n1 + 7) / 8 * 8 * pl->n2;
+  }
   return 0;
 }
 
@@ -716,6 +722,11 @@ static int run_fft_f32(soi_desc_t *d, soi_plan_t *pl, soi_c32_t *X, SoiBatch b, 
     else
       KCHK(soik_fft_single_f32(at, X, pl->tw1_32, winv, pl->Mh, pl->M, S, pl->single_count, b, st));
     mark(pl, 3, st);
+  } else if (pl->fft_longd) {
+    KCHK(soik_fft_longd_cols(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
+                             S, tb, pl->Mt, b, st));
+    mark(pl, 3, st);
+    KCHK(soik_fft_longd_rows(tb, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Mt, pl->M, S, b, st));
   } else if (pl->fft_long && pl->fft_reg) {
     KCHK(soik_fft_long32_cols(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
                               S, pl->cvar, tb, b, st));

@@ -142,26 +142,116 @@ template <int R, typename C> __device__ __forceinline__ void dft_any(C *a)
 }
 
 // ---------------------------------------------------------------------------------------------
+// The same operations with every fused multiply-add written out, the way the compiler contracts
+// soi_common.hpp's forms in the LDS transform: for results that do not depend on what surrounds them.
+// ---------------------------------------------------------------------------------------------
+namespace pinned {
+#pragma clang fp contract(off)
+__device__ __forceinline__ float fm(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ float2 cmul(float2 a, float2 b)
+{
+  return float2{fm(a.x, b.x, -(a.y * b.y)), fm(a.y, b.x, a.x * b.y)};
+}
+// ... the pass-1 twiddle: the other product of the imaginary part is the rounded one
+__device__ __forceinline__ float2 cmul_t(float2 a, float2 t)
+{
+  return float2{fm(a.x, t.x, -(a.y * t.y)), fm(a.x, t.y, a.y * t.x)};
+}
+__device__ __forceinline__ void dft3(float2 *a)
+{
+  const float h = 0.86602540378443864676f;
+  const float2 t = cadd(a[1], a[2]), d = csub(a[1], a[2]);
+  const float2 m = float2{fm(-0.5f, t.x, a[0].x), fm(-0.5f, t.y, a[0].y)};
+  a[0] = cadd(a[0], t);
+  a[1] = float2{fm(h, d.y, m.x), fm(-h, d.x, m.y)};
+  a[2] = float2{fm(-h, d.y, m.x), fm(h, d.x, m.y)};
+}
+__device__ __forceinline__ void dft5(float2 *a)
+{
+  const float c1 = 0.30901699437494742410f, c2 = -0.80901699437494742410f;
+  const float s1 = 0.95105651629515357212f, s2 = 0.58778525229247312917f;
+  const float2 b1 = cadd(a[1], a[4]), b2 = cadd(a[2], a[3]);
+  const float2 d1 = csub(a[1], a[4]), d2 = csub(a[2], a[3]), x0 = a[0];
+  const float2 p1 = float2{fm(c2, b2.x, fm(c1, b1.x, x0.x)), fm(c2, b2.y, fm(c1, b1.y, x0.y))};
+  const float2 p2 = float2{fm(c1, b2.x, fm(c2, b1.x, x0.x)), fm(c1, b2.y, fm(c2, b1.y, x0.y))};
+  const float2 q1 = float2{fm(s2, d2.x, s1 * d1.x), fm(s2, d2.y, s1 * d1.y)};
+  const float2 q2 = float2{fm(s2, d1.x, -(s1 * d2.x)), fm(s2, d1.y, -(s1 * d2.y))};
+  a[0] = cadd(cadd(x0, b1), b2);
+  a[1] = float2{p1.x + q1.y, p1.y - q1.x};
+  a[4] = float2{p1.x - q1.y, p1.y + q1.x};
+  a[2] = float2{p2.x + q2.y, p2.y - q2.x};
+  a[3] = float2{p2.x - q2.y, p2.y + q2.x};
+}
+__device__ __forceinline__ void dft8(float2 *a)
+{
+  const float r = 0.70710678118654752440f;
+  dft4(a[0], a[2], a[4], a[6]);
+  dft4(a[1], a[3], a[5], a[7]);
+  const float2 e0 = a[0], e1 = a[2], e2 = a[4], e3 = a[6], o0 = a[1], o2 = cmul_mi(a[5]);
+  const float s1 = a[3].x + a[3].y, d1 = a[3].y - a[3].x, d3 = a[7].y - a[7].x, s3 = a[7].x + a[7].y;
+  a[0] = cadd(e0, o0);
+  a[4] = csub(e0, o0);
+  a[1] = float2{fm(r, s1, e1.x), fm(r, d1, e1.y)};
+  a[5] = float2{fm(-r, s1, e1.x), fm(-r, d1, e1.y)};
+  a[2] = cadd(e2, o2);
+  a[6] = csub(e2, o2);
+  a[3] = float2{fm(r, d3, e3.x), fm(-r, s3, e3.y)};
+  a[7] = float2{fm(-r, d3, e3.x), fm(r, s3, e3.y)};
+}
+template <int R> __device__ __forceinline__ void dft_any(float2 *a)
+{
+  if constexpr (R == 3) dft3(a);
+  else if constexpr (R == 5) dft5(a);
+  else if constexpr (R == 8) dft8(a);
+  else dft_r<R>(a);  // 2, 4: additions only
+}
+}  // namespace pinned
+
+// by FORM (see Sched): products and DFTs as the compiler fuses them, or pinned
+template <int FORM, typename C> __device__ __forceinline__ C cmul_as(C a, C b)
+{
+  if constexpr (FORM == 0) return cmul(a, b);
+  else return pinned::cmul(a, b);
+}
+template <int FORM, int R, typename C> __device__ __forceinline__ void dft_as(C *a)
+{
+  if constexpr (FORM == 0) dft_any<R>(a);
+  else pinned::dft_any<R>(a);
+}
+
+// ---------------------------------------------------------------------------------------------
 // compile-time schedule of one transform: L points, TS threads per sequence, radices in stage
 // order.  Stage s has L/R butterflies; thread ts takes butterflies ts, ts + TS, ...
 // ---------------------------------------------------------------------------------------------
+//
+// A stage may be a chain of radices that run one after the other in registers: two decimal digits
+// for each, the first in front (20503 = radix 2, then 5, then 3: 30 values, all twiddles of the
+// three stages from the table).  FORM says how twiddles are made and which DFTs are used:
+//   0: powers of a few table reads (see chain), products of coprime factors without twiddles;
+//   2: every twiddle from the table, as soi_common.hpp's LDS transform does.
+// ---------------------------------------------------------------------------------------------
+constexpr int code_prod(int c) { return c < 100 ? c : c % 100 * code_prod(c / 100); }
+constexpr int code_first(int c) { return c < 100 ? c : code_first(c / 100); }
+constexpr int code_rest(int c) { return c < 100 ? 0 : c % 100 + 100 * code_rest(c / 100); }
+
 template <int L_, int TS_, int... Rs> struct Sched {
-  static constexpr int L = L_, TS = TS_, n = sizeof...(Rs);
+  static constexpr int L = L_, TS = TS_, n = sizeof...(Rs), FORM = 0;
   static constexpr int r[n] = {Rs...};
-  static constexpr int at(int s) { return r[s]; }
+  static constexpr int code(int s) { return r[s]; }
+  static constexpr int at(int s) { return code_prod(r[s]); }
   static constexpr int span(int s)  // product of radices before stage s
   {
     int p = 1;
-    for (int i = 0; i < s; ++i) p *= r[i];
+    for (int i = 0; i < s; ++i) p *= at(i);
     return p;
   }
-  static constexpr int nb(int s) { return L / r[s]; }                      // butterflies
+  static constexpr int nb(int s) { return L / at(s); }                     // butterflies
   static constexpr int nc(int s) { return (nb(s) + TS - 1) / TS; }         // rounds per thread
   static constexpr int e()                                                 // values per thread
   {
     int m = 0;
     for (int s = 0; s < n; ++s)
-      if (nc(s) * r[s] > m) m = nc(s) * r[s];
+      if (nc(s) * at(s) > m) m = nc(s) * at(s);
     return m;
   }
   static constexpr int E = e();
@@ -169,6 +259,7 @@ template <int L_, int TS_, int... Rs> struct Sched {
   // the same transform on at most N threads
   template <int N> using Cap = Sched<L_, (TS_ < N ? TS_ : N), Rs...>;
 };
+template <int F, typename SC> struct WithForm : SC { static constexpr int FORM = F; };
 
 // LDS position of element pos of a sequence.  The first stage's threads write R0 positions apart.
 // When R0 is a power of two those fall on the same banks, unless a position covers all of them
@@ -252,40 +343,68 @@ __device__ __forceinline__ void exchange(C (&v)[SC::E], unsigned char *lds, int 
 
 constexpr int bit_len(int x) { return x ? 1 + bit_len(x >> 1) : 0; }
 
-// twiddle + DFT of every butterfly of stage S0 held in registers.  The R - 1 twiddles w^k of a
-// butterfly come from the log2 R table reads w^(2^b): w^k is the product of the powers of k's
-// set bits (at most three extra roundings for R = 16), so a thread issues a few loads per
-// butterfly instead of R - 1.
+// The radices of CODE on the values v of one butterfly: input k is position j + k*L/R, output k goes to
+// position k*NS of the butterfly's outputs, jm = j % NS.  The first radix R1 of the chain has R/R1
+// butterflies with the same jm; its output k continues, by itself, with jm + k*NS at span NS*R1.
+// FORM < 2: the R1 - 1 twiddles w^k of a butterfly come from the log2 R1 table reads w^(2^b): w^k is
+// the product of the powers of k's set bits (at most three extra roundings for R1 = 16), so a
+// thread issues a few loads per butterfly instead of R1 - 1.
+template <int FORM, int L, int NS, int CODE, typename C>
+__device__ __forceinline__ void chain(C *v, int jm, const C *__restrict__ tw)
+{
+  constexpr int R1 = code_first(CODE), REST = code_rest(CODE), M = REST ? code_prod(REST) : 1;
+  constexpr int NBITS = bit_len(R1 - 1), step = L / (NS * R1);
+  C w[R1];
+  if constexpr (NS > 1 && FORM < 2) {
+    C p[NBITS];
+#pragma unroll
+    for (int b = 0; b < NBITS; ++b) p[b] = tw[(jm * step) << b];
+#pragma unroll
+    for (int k = 1; k < R1; ++k) {
+      bool first = true;
+#pragma unroll
+      for (int b = 0; b < NBITS; ++b)
+        if (k & (1 << b)) {
+          w[k] = first ? p[b] : cmul_as<FORM>(w[k], p[b]);
+          first = false;
+        }
+    }
+  } else if constexpr (NS > 1) {
+#pragma unroll
+    for (int k = 1; k < R1; ++k) w[k] = tw[k * jm * step];
+  }
+  C u[R1][M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    C a[R1];
+#pragma unroll
+    for (int k = 0; k < R1; ++k) a[k] = v[i + k * M];
+    if constexpr (NS > 1) {
+#pragma unroll
+      for (int k = 1; k < R1; ++k) a[k] = cmul_as<FORM>(a[k], w[k]);
+    }
+    dft_as<FORM, R1>(a);
+#pragma unroll
+    for (int k = 0; k < R1; ++k) u[k][i] = a[k];
+  }
+#pragma unroll
+  for (int k = 0; k < R1; ++k) {
+    if constexpr (REST != 0) chain<FORM, L, NS * R1, REST>(u[k], jm + k * NS, tw);
+#pragma unroll
+    for (int i = 0; i < M; ++i) v[k + R1 * i] = u[k][i];
+  }
+}
+
+// twiddle + DFT of every butterfly of stage S0 held in registers
 template <typename SC, int S0, typename C>
 __device__ __forceinline__ void stage(C (&v)[SC::E], int ts, const C *__restrict__ tw)
 {
   constexpr int TS = SC::TS, R = SC::at(S0), NS = SC::span(S0), NB = SC::nb(S0), NC = SC::nc(S0);
-  constexpr int NBITS = bit_len(R - 1);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int j = ts + TS * c;
-    if ((c + 1) * TS <= NB || j < NB) {
-      if constexpr (NS > 1) {
-        const int jm = j % NS;
-        constexpr int step = SC::L / (NS * R);
-        C p[NBITS];
-#pragma unroll
-        for (int b = 0; b < NBITS; ++b) p[b] = tw[(jm * step) << b];
-#pragma unroll
-        for (int k = 1; k < R; ++k) {
-          C w = C{0, 0};
-          bool first = true;
-#pragma unroll
-          for (int b = 0; b < NBITS; ++b)
-            if (k & (1 << b)) {
-              w = first ? p[b] : cmul(w, p[b]);
-              first = false;
-            }
-          v[c * R + k] = cmul(v[c * R + k], w);
-        }
-      }
-      dft_any<R>(&v[c * R]);
-    }
+    if ((c + 1) * TS <= NB || j < NB)
+      chain<SC::FORM, SC::L, NS, SC::code(S0)>(&v[c * R], NS > 1 ? j % NS : 0, tw);
   }
 }
 
@@ -378,36 +497,54 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_cols(
     }
   }
 
+  // FORM 2 reads a pair for each value, and the lanes' entries of the lower table lie all over it (up
+  // to 64 cache lines an instruction, 60% of the L1's cycles): a copy in LDS (1440 points: 199 against
+  // 226 us)
+  [[maybe_unused]] C *llo = reinterpret_cast<C *>(lds_raw + fft_lds<SC, T, FULL, C>());
+  if constexpr (SC::FORM == 2)
+    for (int e = tid; e < 1 << lb1; e += T * TS) llo[e] = tlo[e];
+
   run_stages<SC, T, FULL, 0, C>(v, lds_raw, q, ts, tw);
 
   // twiddle w_Mhat^{r2 m1}, m1 = j + k*L/RL, from the two-level table (hi[e >> lb1] *
   // lo[e & mask], exponents below M_hat < 2^32), factored into w^{r2 j} w^{r2 k L/RL}: a thread
-  // reads NC + RL - 1 table pairs instead of NC * RL
+  // reads NC + RL - 1 table pairs instead of NC * RL (FORM 2: unfactored)
   constexpr int RL = SC::at(SC::n - 1), NC = SC::nc(SC::n - 1), NB = SC::nb(SC::n - 1);
+  constexpr bool FACT = SC::FORM < 2;
   const unsigned lmask = (1u << lb1) - 1;
   if (!on) return;  // no barrier follows
   C tc[NC];
+  if constexpr (FACT)
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int j = ts + TS * c;
     if ((c + 1) * TS <= NB || j < NB) {
       const unsigned ex = r2 * (unsigned)j;
-      tc[c] = cmul(thi[ex >> lb1], tlo[ex & lmask]);
+      tc[c] = cmul_as<SC::FORM>(thi[ex >> lb1], tlo[ex & lmask]);
     }
   }
   C *tseg = TILED ? tout + (long)s * Mt : nullptr;
 #pragma unroll
   for (int k = 0; k < RL; ++k) {
     C tk = C{1, 0};
-    if (k) {
+    if (FACT && k) {
       const unsigned ex = r2 * (unsigned)(k * (L / RL));
-      tk = cmul(thi[ex >> lb1], tlo[ex & lmask]);
+      tk = cmul_as<SC::FORM>(thi[ex >> lb1], tlo[ex & lmask]);
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int j = ts + TS * c;
       if ((c + 1) * TS <= NB || j < NB) {
-        const C y = cmul(v[c * RL + k], k ? cmul(tc[c], tk) : tc[c]);
+        C t;
+        if constexpr (FACT) {
+          t = k ? cmul_as<SC::FORM>(tc[c], tk) : tc[c];
+        } else {
+          const unsigned ex = r2 * (unsigned)(j + k * (L / RL));
+          t = cmul_as<SC::FORM>(thi[ex >> lb1], llo[ex & lmask]);
+        }
+        C y;
+        if constexpr (SC::FORM == 2) y = pinned::cmul_t(v[c * RL + k], t);
+        else y = cmul_as<SC::FORM>(v[c * RL + k], t);
         if constexpr (TILED && (L / RL) % TR == 0) {  // j + k*L/RL: k moves whole tiles
           const unsigned off = (((unsigned)j / TR * n2s + r2) * TR + (unsigned)j % TR) * (unsigned)sizeof(C);
           st_at(tseg + (size_t)(k * (L / RL)) * n2s, off, y);
@@ -467,9 +604,10 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_rows(
   run_stages<SC, T, FULL, 0, C>(v, lds_raw, q, ts, tw);
 
   // W_inv in FP64, loaded a few at a time ahead of the stores that use them (index clamped, so
-  // that the loads need no branch)
+  // that the loads need no branch); more where the launch leaves each thread the registers
+  // (complex64, 1536 points in blocks of 512 threads: 189 against 204 us; with less room they spill)
   constexpr int RL = SC::at(SC::n - 1), NC = SC::nc(SC::n - 1), NB = SC::nb(SC::n - 1);
-  constexpr int GW = 4;
+  constexpr int GW = sizeof(C) == 8 && MW <= 3 ? 8 : 4;
   if (!on) return;  // no barrier follows
   C *out = X + (long)s * M;
   const unsigned Ml = (unsigned)M;
@@ -560,9 +698,11 @@ static int launch_cols(C *data, const C *tw, const C *thi, const C *tlo, int n2,
 {
   constexpr bool TILED = sizeof(C) == 8;  // complex64: into the row pass's tiles
   auto kern = k_fft_cols<SC, T, FULL, C, TILED, fft_minw<SC, T, FULL, C>()>;
-  constexpr size_t lds = fft_lds<SC, T, FULL, C>();
-  static_assert(lds <= 160 * 1024 && T * SC::TS <= 1024, "tile");
-  static bool once = (allow_lds(kern, lds), true);
+  constexpr size_t base = fft_lds<SC, T, FULL, C>();
+  static_assert(base <= 160 * 1024 && T * SC::TS <= 1024, "tile");
+  const size_t lds = base + (SC::FORM == 2 ? sizeof(C) << lb1 : 0);
+  if (lds > 160 * 1024) return (int)hipErrorInvalidValue;
+  static bool once = (allow_lds(kern, SC::FORM == 2 ? 160 * 1024 : base), true);
   (void)once;
   hipLaunchKernelGGL(kern, dim3((unsigned)((n2 + T - 1) / T * S), b.n > 0 ? b.n : 1),
                      dim3(T * SC::TS), lds, st, data, tw, thi, tlo, n2, lb1, Mh, S, tout, Mt, b);
@@ -581,7 +721,11 @@ static int launch_rows(const C *data, C *X, const C *tw, const double2 *winv, in
   // (512 x 512, 32 segments); 0.58 against 0.64 ms where W_inv is 64 MB (2560 x 2048); elsewhere
   // one by one (1024 x 1024, 64 segments: 0.46 against 0.51 ms).
   const bool cached = (double)S * Mh * sizeof(C) <= 192e6;
-  const int sg = cached ? S : M >= (1L << 21) ? (S < 16 ? S : 16) : 1;
+  // (complex64 FORM 2, whose W_inv entries are twice its values: four together, 133 against 144 us
+  // at 1024 x 960, 32 segments.)
+  const int sg = SC::FORM == 2 ? (S < 4 ? S : 4)
+                 : cached      ? S
+                               : M >= (1L << 21) ? (S < 16 ? S : 16) : 1;
   auto kern = k_fft_rows<SC, T, FULL, C, TILED, fft_minw<SC, T, FULL, C>()>;
   constexpr size_t lds = fft_lds<SC, T, FULL, C>();
   static_assert(lds <= 160 * 1024 && T * SC::TS <= 1024, "tile");

@@ -104,6 +104,13 @@ int soik_fft_long32_cols(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t 
 int soik_fft_long32_rows(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
                          const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S, SoiBatch b,
                          hipStream_t st);
+/* ... of lengths outside that file's list (soi_fft_long32d.hip), columns (rows = 0) or rows (1) */
+int soik_fft_longd_supported(int L, int rows);
+int soik_fft_longd_cols(float2 *data, const float2 *tw1, const float2 *thi, const float2 *tlo, int n1,
+                        int n2, int lb1, long Mh, int S, float2 *tout, long Mt, SoiBatch b,
+                        hipStream_t st);
+int soik_fft_longd_rows(const float2 *data, float2 *X, const float2 *tw2, const double2 *winv, int n1,
+                        int n2, long Mt, long M, int S, SoiBatch b, hipStream_t st);
 int soik_max_exponent(const double *x, int len, int nchunk, int *out, hipStream_t st);
 int soik_compress(int *out, long stride, const double *x, int len, int nchunk, int e_max,
                   const int *emi, int *nwords, const int *e_max_dev, hipStream_t st);
