@@ -106,11 +106,12 @@ int soik_fft_long32_rows(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *t
                          hipStream_t st);
 /* ... of lengths outside that file's list (soi_fft_long32d.hip), columns (rows = 0) or rows (1) */
 int soik_fft_longd_supported(int L, int rows);
-int soik_fft_longd_cols(float2 *data, const float2 *tw1, const float2 *thi, const float2 *tlo, int n1,
-                        int n2, int lb1, long Mh, int S, float2 *tout, long Mt, SoiBatch b,
+int soik_fft_longd_cols(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi,
+                        const soi_c32_t *tlo, int n1, int n2, int lb1, long Mh, int S,
+                        soi_c32_t *tout, long Mt, SoiBatch b, hipStream_t st);
+int soik_fft_longd_rows(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
+                        const soi_c64_t *winv, int n1, int n2, long Mt, long M, int S, SoiBatch b,
                         hipStream_t st);
-int soik_fft_longd_rows(const float2 *data, float2 *X, const float2 *tw2, const double2 *winv, int n1,
-                        int n2, long Mt, long M, int S, SoiBatch b, hipStream_t st);
 int soik_max_exponent(const double *x, int len, int nchunk, int *out, hipStream_t st);
 int soik_compress(int *out, long stride, const double *x, int len, int nchunk, int e_max,
                   const int *emi, int *nwords, const int *e_max_dev, hipStream_t st);
@@ -126,6 +127,7 @@ int soik_compress_flat(int *out, long stride, const double *x, int len, int nchu
                        const int *e_max_dev, const int *emi, const long *unused, hipStream_t st);
 int soik_decompress_flat(double *out, const int *in, long stride, int len, int nchunk,
                          const int *e_max_dev, const int *emi, hipStream_t st);
+int soik_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
 int soik_gen_uniform(soi_c64_t *x, long N, uint64_t seed, hipStream_t st);
 int soik_gen_tones(soi_c64_t *x, long N, const double *tf, const double *tph, int ntones,
                    double amp, double noise_sigma, uint64_t seed, hipStream_t st);

@@ -564,6 +564,15 @@ __global__ __launch_bounds__(256) void k_vlc_exchange(int *__restrict__ out, lon
   }
 }
 
+// Copy between device and pinned host memory, 16-byte units.  A kernel follows the kernels before it in
+// the stream directly, where a DMA engine's copy waits for a signal between queues.
+__global__ __launch_bounds__(256) void k_copy(double2 *__restrict__ dst,
+                                              const double2 *__restrict__ src, long n)
+{
+  const long nt = (long)gridDim.x * blockDim.x;
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += nt) dst[e] = src[e];
+}
+
 // =============================================================================================
 // Synthetic inputs (seeded, counter based) for tests and the benchmark
 // =============================================================================================
@@ -906,6 +915,15 @@ extern "C" int soik_decompress_flat(double *out, const int *in, long stride, int
                                     const int *e_max_dev, const int *emi, hipStream_t st)
 {
   return soik_decompress(out, in, stride, len, nchunk, 0, emi, e_max_dev, st);
+}
+
+extern "C" int soik_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+  if (bytes % 16) return (int)hipErrorInvalidValue;
+  const unsigned nb = nblk((long)(bytes / 16), 256);
+  hipLaunchKernelGGL(k_copy, dim3(nb < 1024 ? nb : 1024), dim3(256), 0, st, (double2 *)dst,
+                     (const double2 *)src, (long)(bytes / 16));
+  return (int)hipGetLastError();
 }
 
 extern "C" int soik_gen_uniform(double2 *x, long N, uint64_t seed, hipStream_t st)
