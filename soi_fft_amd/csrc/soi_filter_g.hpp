@@ -26,11 +26,15 @@
 // (complex taps) or 32 (real), so there they stream from L2 a few K steps ahead; the rows of all lanes
 // exceed LDS at S = 64, so lanes go through in groups of 16.  Two row buffers alternate, one filling
 // (direct-to-LDS loads) while the other is multiplied; results of all groups stay in registers until
-// the S-point DFT.  Measured, VALU form -> here: S = 64, mu = 8/7, N = 7*2^23 1.91 -> 0.95 ms (the
+// the S-point DFT.  Long transforms of S = 32 with resident real taps have four
+// buffers of eight lanes instead (QUAD): with two, the wait for a group's rows covers the stores of the
+// tile before, which share their queue.  N = 2^27 1.34 -> 1.24 ms, 2^26 685 -> 632 us, 2^22 57.7 -> 54.9;
+// it loses where one product chain a wave does not fill the matrix pipe or there is little to multiply
+// (S = 16, N = 2^24 173 -> 187; B = 30, S = 32 157 -> 179).  Measured, VALU form -> here: S = 64, mu = 8/7, N = 7*2^23 1.91 -> 0.95 ms (the
 // products alone: 0.55); S = 32, mu = 8/7, N = 7*2^20 190 -> 111 us; B = 44, N = 2^22, S = 16 88 ->
 // 54; S = 64, N = 2^24 305 -> 230.  Against rows in a ring that only the new rows of a tile entered
 // (real taps, S <= 32): N = 2^22, S = 4 59 -> 49 us, S = 8 56 -> 48, S = 16 56 -> 50, S = 32 58 -> 56;
-// N = 2^27, S = 32 1.33 ms either way (products 0.73, memory 0.85).
+// N = 2^27, S = 32 1.33 ms either way (products 0.73, memory 0.85; two buffers).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -43,7 +47,7 @@ namespace soi {
 typedef double gd4 __attribute__((ext_vector_type(4)));
 typedef double gd2 __attribute__((ext_vector_type(2)));
 
-template <int S_, int NMU_, int DMU_, int NK_, bool CT_> struct FilterG {
+template <int S_, int NMU_, int DMU_, int NK_, bool CT_, bool QUAD_ = false> struct FilterG {
   static constexpr int S = S_, NMU = NMU_, DMU = DMU_, NK = NK_;
   static constexpr bool CT = CT_;
   static constexpr int ND = NMU == 5 ? 3 : 2;    // row groups side by side in the columns
@@ -51,11 +55,15 @@ template <int S_, int NMU_, int DMU_, int NK_, bool CT_> struct FilterG {
   static constexpr int TJ = 8 * ND;              // row groups per tile
   static constexpr int MS = ND * DMU;            // input rows from m to m + 1
   static constexpr int ROWS = 7 * MS + 4 * NK;   // input rows per tile
-  static constexpr int GL = S < 16 ? S : 16;     // lanes per group
-  static constexpr int NGRP = S / GL;
-  static constexpr int NW = S < 16 ? S / 2 : 8;  // waves; two lanes of a group each
-  static constexpr int T = NW * 64;
+  static constexpr int NW = S < 16 ? S / 2 : 8;  // waves
   static constexpr int LPW = S / NW;             // lanes i = NW li + w of a wave, li < LPW
+  // B operands resident in registers, or streamed
+  static constexpr bool RES = LPW * NK * (CT ? 4 : 2) <= 160;
+  static constexpr bool QUAD = QUAD_;            // four row buffers of eight lanes, not two
+  static constexpr int NBUF = QUAD ? 4 : 2;
+  static constexpr int GL = S < 16 ? S : QUAD ? 8 : 16;  // lanes per group: GL / NW a wave
+  static constexpr int NGRP = S / GL;
+  static constexpr int T = NW * 64;
   static constexpr int RPC = 64 / GL;            // rows per chunk (64 values, one wave-wide load)
   static constexpr int NCHK = (ROWS + RPC - 1) / RPC;
   static constexpr int NLD = (NCHK + NW - 1) / NW;   // loads per wave and buffer
@@ -66,13 +74,12 @@ template <int S_, int NMU_, int DMU_, int NK_, bool CT_> struct FilterG {
   static constexpr int GP = S + 1;
   static constexpr int NTASK = GRH * LPW;
   static constexpr int NC = (NTASK + T - 1) / T;
-  // B operands resident in registers, or streamed
-  static constexpr bool RES = LPW * NK * (CT ? 4 : 2) <= 160;
   static constexpr int NB = 64 / (4 * GL);       // A address bases (K steps per chunk)
-  static constexpr int LDS_BYTES = (2 * NCHK * CP + GRH * GP + S + (CT ? 1 : NMU * S)) * 16;
+  static constexpr int LDS_BYTES = (NBUF * NCHK * CP + GRH * GP + S + (CT ? 1 : NMU * S)) * 16;
   static constexpr int MIN_M = NCHK * RPC;       // rows of a tile's loads wrap at most once
   static_assert(NK % 2 == 0 || CT, "real taps are loaded two K steps at a time");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
+  static_assert(!QUAD || (RES && !CT && S >= 16 && NC == 1), "four buffers");
 };
 
 // Products with the fused operations spelled out and an 8-point DFT with none: a tile's results are
@@ -124,19 +131,29 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
   x = batch_ptr(x, b.x);
   at = batch_ptr(at, b.at);
   ggd2 *const atg = (ggd2 *)at;
-  __shared__ __align__(16) double2 buf0[F::NCHK * F::CP];
-  __shared__ __align__(16) double2 buf1[F::NCHK * F::CP];
+  // (buffers of their own names: the compiler then knows which loads an LDS read has to wait for)
+  constexpr int BSZ = F::NCHK * F::CP;
+  __shared__ __align__(16) double2 buf0[BSZ];
+  __shared__ __align__(16) double2 buf1[BSZ];
+  __shared__ __align__(16) double2 buf2[F::QUAD ? BSZ : 1];
+  __shared__ __align__(16) double2 buf3[F::QUAD ? BSZ : 1];
   __shared__ __align__(16) double2 G[F::GRH * GP];
   __shared__ __align__(16) double2 tw[S];
   __shared__ __align__(16) double2 pfl[CT ? 1 : F::NMU * S];
+  auto rows_buf = [&](int i) __attribute__((always_inline)) -> double2 * {
+    return i == 0 ? buf0 : i == 1 ? buf1 : i == 2 ? buf2 : buf3;
+  };
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
 
   const long ntiles = (nJ + F::TJ - 1) / F::TJ;
-  const long t0 = (long)blockIdx.x * tiles_per_block;
-  const long t1 = min(ntiles, t0 + tiles_per_block);
-  if (t0 >= t1) return;
+  // tiles t0, t0 + step, ..., t1.  QUAD: the blocks go through the tiles side by side, so that what
+  // they load and store at a time is adjacent
+  const long step = F::QUAD ? gridDim.x : 1;
+  const long t0 = F::QUAD ? xcd_remap(blockIdx.x, gridDim.x) : (long)blockIdx.x * tiles_per_block;
+  if (t0 >= ntiles) return;
+  const long t1 = F::QUAD ? t0 + (ntiles - 1 - t0) / step * step : min(ntiles, t0 + tiles_per_block) - 1;
 
   // rows of lane group gr of a tile into a buffer: element e of the tile's rows (row e / GL, place
   // e % GL) at LDS place e + e / 64.  With 16 lanes a row is all the banks of an 8-byte read, so odd
@@ -157,6 +174,10 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
     }
   };
   dma(buf0, t0, 0);
+  if constexpr (F::QUAD) {
+    dma(buf1, t0, 1);
+    dma(buf2, min(t0 + 2 / NGRP * step, t1), 2 % NGRP);
+  }
 
   for (int e = tid; e < S; e += F::T) tw[e] = twS[e];
   if constexpr (!CT)
@@ -216,10 +237,27 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
 
   double2 gam[LPW][2];  // [li][h]: row m = 4h + g, column n
 
+  auto wait_loads = [&](auto n_tag) __attribute__((always_inline)) {  // all but the last n vector memory operations
+    constexpr int N = decltype(n_tag)::value;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | (N >> 4 << 14));
+  };
   // MFMA of lane group gr from buf
   auto mul = [&](const double2 *buf, auto gr_tag) __attribute__((always_inline)) {
     constexpr int gr = decltype(gr_tag)::value, ng = (gr + 1) % NGRP;
-    if constexpr (CT) {
+    if constexpr (F::QUAD) {
+      gd4 cr = {0, 0, 0, 0};
+      double a[3] = {aread(buf, 0, 0), aread(buf, 0, 1)};
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) {
+        const double2 w = wb[gr][ks / 2];
+        if (ks + 2 < NK) a[(ks + 2) % 3] = aread(buf, 0, ks + 2);
+        cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks % 3], ks & 1 ? w.y : w.x, cr, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) gam[gr][h] = double2{cr[h], cr[h + 2]};
+    } else if constexpr (CT) {
 #pragma unroll
       for (int lh = 0; lh < 2; ++lh) {
         gd4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
@@ -274,62 +312,79 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
     }
   };
 
-  // S-point DFT and stores of a tile.  The loads of the next tile's first group (issued before
-  // this tile's last product) are waited for before the stores are issued, so that the wait does not
-  // cover them.
-  auto epilogue = [&](long tile) __attribute__((always_inline)) {
-    const int jrem = (int)min((long)F::TJ, nJ - tile * F::TJ);  // the last tile may hold fewer row groups
+  // S-point DFT and stores of a tile, round rd of the exchange: LPW-point DFTs of the wave's lanes
+  // into G, and NW-point DFTs out of G to HBM.  `wait` runs before the first stores.
+  auto put = [&](int rd) __attribute__((always_inline)) {
     int tv = tid;
     asm volatile("" : "+v"(tv));  // keep the addresses below out of registers in the tile loop
     const int nv = tv & 15, gv = (tv >> 4) & 3;
+#pragma unroll
+    for (int hh = 0; hh < 2 / F::NH; ++hh) {
+      const int h = F::NH == 2 ? rd : hh;
+      double2 v[LPW];
+#pragma unroll
+      for (int li = 0; li < LPW; ++li) {
+        v[li] = gam[li][h];
+        if constexpr (!CT) v[li] = cmul_fma(v[li], pfl[nv % F::NMU * S + NW * li + wave]);
+      }
+      dft_plain<LPW>(v);
+      if (F::NCOL == 16 || nv < F::NCOL) {
+        double2 *gr = G + (F::NCOL * (F::NH == 2 ? gv : 4 * h + gv) + nv) * GP + wave;
+        gr[0] = v[0];
+#pragma unroll
+        for (int s1 = 1; s1 < LPW; ++s1) gr[s1 * NW] = cmul_fma(v[s1], tw[(wave * s1) % S]);
+      }
+    }
+  };
+  auto get = [&](int rd, long tile, auto wait) __attribute__((always_inline)) {
+    const int jrem = (int)min((long)F::TJ, nJ - tile * F::TJ);  // the last tile may hold fewer row groups
+    int tv = tid;
+    asm volatile("" : "+v"(tv));
     const long R0 = tile * F::GR;
 #pragma unroll
+    for (int c = 0; c < F::NC; ++c) {
+      const int e = tv + c * F::T;
+      const int r = e % F::GRH, s1 = e / F::GRH;
+      double2 u[NW];
+      const bool on = (c + 1) * F::T <= F::NTASK || e < F::NTASK;
+      if (on) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) u[w] = G[r * GP + s1 * NW + w];
+        dft_plain<NW>(u);
+      }
+      if (c == 0) wait();
+      if (on && (rd * F::GRH + r) / F::NMU < jrem) {
+#pragma unroll
+        for (int s2 = 0; s2 < NW; ++s2)
+          __builtin_nontemporal_store(gd2{u[s2].x, u[s2].y},
+                                      atg + (long)(s1 + LPW * s2) * Mh + R0 + rd * F::GRH + r);
+      }
+    }
+  };
+  typedef std::integral_constant<int, 0> zero;
+  // The loads of the next tile's first group (issued before this tile's last product) are waited for
+  // before the stores are issued, so that the wait does not cover them.
+  auto epilogue = [&](long tile) __attribute__((always_inline)) {
+#pragma unroll
     for (int rd = 0; rd < F::NH; ++rd) {
-#pragma unroll
-      for (int hh = 0; hh < 2 / F::NH; ++hh) {
-        const int h = F::NH == 2 ? rd : hh;
-        double2 v[LPW];
-#pragma unroll
-        for (int li = 0; li < LPW; ++li) {
-          v[li] = gam[li][h];
-          if constexpr (!CT) v[li] = cmul_fma(v[li], pfl[nv % F::NMU * S + NW * li + wave]);
-        }
-        dft_plain<LPW>(v);
-        if (F::NCOL == 16 || nv < F::NCOL) {
-          double2 *gr = G + (F::NCOL * (F::NH == 2 ? gv : 4 * h + gv) + nv) * GP + wave;
-          gr[0] = v[0];
-#pragma unroll
-          for (int s1 = 1; s1 < LPW; ++s1) gr[s1 * NW] = cmul_fma(v[s1], tw[(wave * s1) % S]);
-        }
-      }
+      put(rd);
       lds_barrier();
-#pragma unroll
-      for (int c = 0; c < F::NC; ++c) {
-        const int e = tv + c * F::T;
-        const int r = e % F::GRH, s1 = e / F::GRH;
-        double2 u[NW];
-        const bool on = (c + 1) * F::T <= F::NTASK || e < F::NTASK;
-        if (on) {
-#pragma unroll
-          for (int w = 0; w < NW; ++w) u[w] = G[r * GP + s1 * NW + w];
-          dft_plain<NW>(u);
-        }
-        if (rd == 0 && c == 0) {
-          asm volatile("" ::: "memory");
-          __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0)
-        }
-        if (on && (rd * F::GRH + r) / F::NMU < jrem) {
-#pragma unroll
-          for (int s2 = 0; s2 < NW; ++s2)
-            __builtin_nontemporal_store(gd2{u[s2].x, u[s2].y},
-                                        atg + (long)(s1 + LPW * s2) * Mh + R0 + rd * F::GRH + r);
-        }
-      }
+      get(rd, tile, [&]() __attribute__((always_inline)) { if (rd == 0) wait_loads(zero{}); });
       lds_barrier();  // G is free; after the last round the next tile's rows are complete too
     }
   };
 
-  // one tile; its group 0 is in buf0 (BUF = 0) or buf1
+  // One tile, its group 0 in buffer BUF.
+  //
+  // Two buffers: the next group's rows load while a group is multiplied.
+  //
+  // Four (QUAD): rows load three groups ahead, and a group's end waits for the next group's rows only:
+  // the two groups loaded after them stay in flight, and so do the stores of a tile that were issued
+  // since (the waves that store issue all NW of them, but for the last tile of all, which nothing
+  // follows).  One barrier a group: the last one also covers G, which the next tile's put, a barrier
+  // or more later, overwrites; a wave that has stored goes on to the next product by itself.
+  constexpr int NL = F::NLD;
+  const bool stores = wave * 64 < F::NTASK;
   auto body = [&](long tile, auto buf_tag) __attribute__((always_inline)) {
     constexpr int BUF = decltype(buf_tag)::value;
     // an opaque table address (in the global address space, or the loads would wait for LDS too):
@@ -337,14 +392,25 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
     // registers
     asm volatile("" : "+s"(wbase));
     auto group = [&](auto gr_tag) __attribute__((always_inline)) {
-      constexpr int gr = decltype(gr_tag)::value, cur = (BUF + gr) & 1;
-      if constexpr (gr + 1 < NGRP) dma(cur ? buf0 : buf1, tile, gr + 1);
-      else if (tile + 1 < t1) dma(cur ? buf0 : buf1, tile + 1, 0);
-      mul(cur ? buf1 : buf0, gr_tag);
-      if constexpr (gr + 1 < NGRP) {
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0): the next group's rows
+      constexpr int gr = decltype(gr_tag)::value, cur = (BUF + gr) % F::NBUF;
+      if constexpr (F::QUAD) {
+        // past the block's last tile its rows again, so that the counts below hold
+        dma(rows_buf((cur + 3) % 4), min(tile + (gr + 3) / NGRP * step, t1), (gr + 3) % NGRP);
+        mul(rows_buf(cur), gr_tag);
+        if constexpr (gr == NGRP - 1) put(0);
+        // the stores of the tile before came after the next rows' loads in groups 0 and 1
+        if (gr < 2 && stores && tile > t0) wait_loads(std::integral_constant<int, 2 * NL + F::NC * NW>{});
+        else wait_loads(std::integral_constant<int, 2 * NL>{});
         lds_barrier();
+        if constexpr (gr == NGRP - 1) get(0, tile, []() {});
+      } else {
+        if constexpr (gr + 1 < NGRP) dma(rows_buf(cur ^ 1), tile, gr + 1);
+        else if (tile < t1) dma(rows_buf(cur ^ 1), tile + step, 0);
+        mul(rows_buf(cur), gr_tag);
+        if constexpr (gr + 1 < NGRP) {
+          wait_loads(zero{});  // the next group's rows
+          lds_barrier();
+        }
       }
     };
     group(std::integral_constant<int, 0>{});
@@ -353,19 +419,20 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
       group(std::integral_constant<int, 2>{});
       group(std::integral_constant<int, 3>{});
     }
-    epilogue(tile);
+    if constexpr (!F::QUAD) epilogue(tile);
   };
 
-  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0)
+  wait_loads(zero{});
   lds_barrier();
-  if constexpr (NGRP > 1) {  // an even number of groups ends in the buffer it began with
-    for (long tile = t0; tile < t1; ++tile) body(tile, std::integral_constant<int, 0>{});
+  if constexpr (NGRP % F::NBUF == 0) {  // a tile ends in the buffer it began with
+    for (long tile = t0; tile <= t1; tile += step) body(tile, zero{});
   } else {
-    for (long tile = t0; tile < t1; tile += 2) {
-      body(tile, std::integral_constant<int, 0>{});
-      if (tile + 1 < t1) body(tile + 1, std::integral_constant<int, 1>{});
+    for (long tile = t0; tile <= t1; tile += 2 * step) {
+      body(tile, zero{});
+      if (tile < t1) body(tile + step, std::integral_constant<int, NGRP>{});
     }
   }
+  if constexpr (F::QUAD) wait_loads(zero{});  // no load may outlive the block's LDS
 }
 
 // B operand table (see k_filter_g): column col = lane % 16 = theta + n_mu D, k = 4 ks + lane / 16,
@@ -397,7 +464,13 @@ template <typename F> static int filter_g_launch(const SoiFilterArgs *a, hipStre
   long nb = a->b.n > 1 ? (512 * per_cu + a->b.n - 1) / a->b.n : 256 * per_cu;
   if (nb > ntiles) nb = ntiles;
   const int tpb = (int)((ntiles + nb - 1) / nb);
-  nb = (ntiles + tpb - 1) / tpb;
+  // four row buffers where blocks walk more than two tiles (S = 32, N = 2^21: 33.5 -> 32.8 us; two tiles,
+  // N = 2^20: 24 with two buffers, 28 with four); the same bits either way
+  if constexpr (!F::QUAD && F::RES && !F::CT && F::S == 32) {
+    using Q = FilterG<F::S, F::NMU, F::DMU, F::NK, F::CT, true>;
+    if (tpb > 2 && Q::MIN_M <= a->M) return filter_g_launch<Q>(a, st);
+  }
+  if (!F::QUAD) nb = (ntiles + tpb - 1) / tpb;
   hipLaunchKernelGGL(k_filter_g<F>, dim3((unsigned)nb, a->b.n > 0 ? a->b.n : 1), dim3(F::T), 0, st,
                      (const double2 *)a->x, (double2 *)a->at, (const double2 *)a->wt,
                      (const double2 *)a->post, (const double2 *)a->twS, a->M, a->Mh, a->nJ, tpb, a->b);

@@ -66,3 +66,10 @@ def test_filter_form(soi, orc, torch_cuda, S, name):
                                       (32, 25600, "ct44"), (64, 31500, "mu87_72")])
 def test_several_tiles_a_block(soi, orc, torch_cuda, S, M, name):
     run(soi, orc, torch_cuda, S, M, WINDOWS[name])
+
+
+@pytest.mark.parametrize("M", [320, 25600, 54000, 81920])
+def test_four_row_buffers(soi, orc, torch_cuda, M):
+    """S = 32, resident real taps: rows load three groups (of four a tile) ahead.  Blocks of one, two,
+    three and four tiles, the last tile a part."""
+    run(soi, orc, torch_cuda, 32, M, WINDOWS["rt72"])
