@@ -227,7 +227,8 @@ template <int FORM, int R, typename C> __device__ __forceinline__ void dft_as(C 
 // A stage may be a chain of radices that run one after the other in registers: two decimal digits
 // for each, the first in front (20503 = radix 2, then 5, then 3: 30 values, all twiddles of the
 // three stages from the table).  FORM says how twiddles are made and which DFTs are used:
-//   0: powers of a few table reads (see chain), products of coprime factors without twiddles;
+//   0: powers of a few table reads (complex128, see chain) or every twiddle from the table
+//      (complex64), products of coprime factors without twiddles;
 //   2: every twiddle from the table, as soi_common.hpp's LDS transform does.
 // ---------------------------------------------------------------------------------------------
 constexpr int code_prod(int c) { return c < 100 ? c : c % 100 * code_prod(c / 100); }
@@ -341,21 +342,24 @@ __device__ __forceinline__ void exchange(C (&v)[SC::E], unsigned char *lds, int 
   }
 }
 
+constexpr int odd_part(int x) { return x % 2 ? x : odd_part(x / 2); }
 constexpr int bit_len(int x) { return x ? 1 + bit_len(x >> 1) : 0; }
 
 // The radices of CODE on the values v of one butterfly: input k is position j + k*L/R, output k goes to
 // position k*NS of the butterfly's outputs, jm = j % NS.  The first radix R1 of the chain has R/R1
 // butterflies with the same jm; its output k continues, by itself, with jm + k*NS at span NS*R1.
-// FORM < 2: the R1 - 1 twiddles w^k of a butterfly come from the log2 R1 table reads w^(2^b): w^k is
-// the product of the powers of k's set bits (at most three extra roundings for R1 = 16), so a
-// thread issues a few loads per butterfly instead of R1 - 1.
+// Complex128 (FORM 0): the R1 - 1 twiddles w^k of a butterfly come from the log2 R1 table reads
+// w^(2^b): w^k is the product of the powers of k's set bits (at most three extra roundings for R1 =
+// 16), so a thread issues a few loads per butterfly instead of R1 - 1.  Complex64 reads each: the
+// products cost 3 to 5% of the transform's error (N = 2^22: 3.34e-7 against 3.18e-7) for 0 to 8% of its
+// time.
 template <int FORM, int L, int NS, int CODE, typename C>
 __device__ __forceinline__ void chain(C *v, int jm, const C *__restrict__ tw)
 {
   constexpr int R1 = code_first(CODE), REST = code_rest(CODE), M = REST ? code_prod(REST) : 1;
   constexpr int NBITS = bit_len(R1 - 1), step = L / (NS * R1);
   C w[R1];
-  if constexpr (NS > 1 && FORM < 2) {
+  if constexpr (NS > 1 && FORM < 2 && sizeof(C) == 16) {
     C p[NBITS];
 #pragma unroll
     for (int b = 0; b < NBITS; ++b) p[b] = tw[(jm * step) << b];
@@ -510,7 +514,10 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_cols(
   // lo[e & mask], exponents below M_hat < 2^32), factored into w^{r2 j} w^{r2 k L/RL}: a thread
   // reads NC + RL - 1 table pairs instead of NC * RL (FORM 2: unfactored)
   constexpr int RL = SC::at(SC::n - 1), NC = SC::nc(SC::n - 1), NB = SC::nb(SC::n - 1);
-  constexpr bool FACT = SC::FORM < 2;
+  // Complex64 factors it only for n1 = F 2^a, F = 1 and 5; elsewhere that would add to its error (N =
+  // 27*2^17: 3.23e-7, unfactored 3.17e-7, the same time).
+  constexpr int ODD = odd_part(L);
+  constexpr bool FACT = SC::FORM < 2 && (sizeof(C) == 16 || ODD == 1 || ODD == 5);
   const unsigned lmask = (1u << lb1) - 1;
   if (!on) return;  // no barrier follows
   C tc[NC];
@@ -540,7 +547,8 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_cols(
           t = k ? cmul_as<SC::FORM>(tc[c], tk) : tc[c];
         } else {
           const unsigned ex = r2 * (unsigned)(j + k * (L / RL));
-          t = cmul_as<SC::FORM>(thi[ex >> lb1], llo[ex & lmask]);
+          const C *lo = SC::FORM == 2 ? llo : tlo;
+          t = cmul_as<SC::FORM>(thi[ex >> lb1], lo[ex & lmask]);
         }
         C y;
         if constexpr (SC::FORM == 2) y = pinned::cmul_t(v[c * RL + k], t);
