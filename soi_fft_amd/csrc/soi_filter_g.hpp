@@ -82,9 +82,9 @@ template <int S_, int NMU_, int DMU_, int NK_, bool CT_, bool QUAD_ = false> str
   static_assert(!QUAD || (RES && !CT && S >= 16 && NC == 1), "four buffers");
 };
 
-// Products with the fused operations spelled out and an 8-point DFT with none: a tile's results are
-// then the same bit for bit in every code copy that the compiler makes (batched launches split the
-// tiles over blocks differently).
+// Products and an 8-point DFT with the fused operations spelled out: a tile's results are then the same bit
+// for bit in every code copy that the compiler makes (batched launches split the tiles over blocks
+// differently).
 __device__ __forceinline__ double2 cmul_fma(double2 a, double2 b)
 {
   return double2{__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x)};
@@ -95,24 +95,25 @@ __device__ __forceinline__ void dft8_plain(double2 *a)
   const double r = 0.70710678118654752440084436210485;
   dft4(a[0], a[2], a[4], a[6]);
   dft4(a[1], a[3], a[5], a[7]);
-  const double2 o1 = double2{r * (a[3].x + a[3].y), r * (a[3].y - a[3].x)};
-  const double2 o2 = cmul_mi(a[5]);
-  const double2 o3 = double2{r * (a[7].y - a[7].x), -r * (a[7].x + a[7].y)};
-  const double2 e0 = a[0], e1 = a[2], e2 = a[4], e3 = a[6];
+  const double2 e0 = a[0], e1 = a[2], e2 = a[4], e3 = a[6], o2 = cmul_mi(a[5]);
+  const double s1 = a[3].x + a[3].y, d1 = a[3].y - a[3].x, d3 = a[7].y - a[7].x, s3 = a[7].x + a[7].y;
   a[0] = double2{e0.x + a[1].x, e0.y + a[1].y};
   a[4] = double2{e0.x - a[1].x, e0.y - a[1].y};
-  a[1] = double2{e1.x + o1.x, e1.y + o1.y};
-  a[5] = double2{e1.x - o1.x, e1.y - o1.y};
+  a[1] = double2{__builtin_fma(r, s1, e1.x), __builtin_fma(r, d1, e1.y)};
+  a[5] = double2{__builtin_fma(-r, s1, e1.x), __builtin_fma(-r, d1, e1.y)};
   a[2] = double2{e2.x + o2.x, e2.y + o2.y};
   a[6] = double2{e2.x - o2.x, e2.y - o2.y};
-  a[3] = double2{e3.x + o3.x, e3.y + o3.y};
-  a[7] = double2{e3.x - o3.x, e3.y - o3.y};
+  a[3] = double2{__builtin_fma(r, d3, e3.x), __builtin_fma(-r, s3, e3.y)};
+  a[7] = double2{__builtin_fma(-r, d3, e3.x), __builtin_fma(r, s3, e3.y)};
 }
 template <int R> __device__ __forceinline__ void dft_plain(double2 *a)
 {
   if constexpr (R == 8) dft8_plain(a);
   else dft_r<R>(a);
 }
+
+// Place q of n in the order from both ends inwards: 0, n - 1, 1, n - 2, ...
+constexpr int inwards(int q, int n) { return q & 1 ? n - 1 - q / 2 : q / 2; }
 
 // B operands of lane i: double2 {Re t, Im t} per K step (complex taps) or two K steps (real)
 template <typename F>
@@ -183,8 +184,18 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
   if constexpr (!CT)
     for (int e = tid; e < F::NMU * S; e += F::T) pfl[e] = post[e];
 
-  // B operand table: item it of lane i at wt[(i * NIT + it) * 64 + lane]
+  // B operand table: item it of lane i at wt[(i * NIT + it) * 64 + lane].  Items are multiplied from the
+  // ends of the taps inwards (item(j) is the j-th; of its two K steps, real taps, the outer one
+  // first): the taps peak in the middle, so a chain's sum stays small until its last steps.  In the
+  // order of the taps every step after the peak rounds the whole sum: S = 16, error of the filter with
+  // 72 real taps 3.8e-16 -> 2.9e-16, with 44 complex 2.5e-16 -> 1.8e-16 (the VALU form, which adds two
+  // or four slices: 1.8e-16).  The time is the same.
   constexpr int NIT = CT ? NK : NK / 2;
+  auto item = [](int j) { return inwards(j, NIT); };
+  auto kstep = [&](int q) {
+    if constexpr (CT) return item(q);
+    else return 2 * item(q / 2) + ((q & 1) ^ (q / 2 & 1));
+  };
   const unsigned lane16 = lane * 16u;
   typedef const __attribute__((address_space(1))) char gchar;
   typedef const __attribute__((address_space(1))) gd2 cgd2;
@@ -207,10 +218,10 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
   static_assert(F::RES || SEQ % PD == 0, "prefetch ring");
   double2 bq[F::RES ? 1 : PD][WID];
   auto bnext = [&](int gr, int it) {  // item it (< SEQ) of group gr into its ring place
-    if constexpr (CT) bq[it % PD][0] = bload(2 * gr + it / NIT, it % NIT);
+    if constexpr (CT) bq[it % PD][0] = bload(2 * gr + it / NIT, item(it % NIT));
     else {
-      bq[it % PD][0] = bload(2 * gr, it);
-      bq[it % PD][WID - 1] = bload(2 * gr + 1, it);
+      bq[it % PD][0] = bload(2 * gr, item(it));
+      bq[it % PD][WID - 1] = bload(2 * gr + 1, item(it));
     }
   };
   if constexpr (!F::RES) {
@@ -247,12 +258,13 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
     constexpr int gr = decltype(gr_tag)::value, ng = (gr + 1) % NGRP;
     if constexpr (F::QUAD) {
       gd4 cr = {0, 0, 0, 0};
-      double a[3] = {aread(buf, 0, 0), aread(buf, 0, 1)};
+      double a[3] = {aread(buf, 0, kstep(0)), aread(buf, 0, kstep(1))};
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) {
+      for (int q = 0; q < NK; ++q) {
+        const int ks = kstep(q);
         const double2 w = wb[gr][ks / 2];
-        if (ks + 2 < NK) a[(ks + 2) % 3] = aread(buf, 0, ks + 2);
-        cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks % 3], ks & 1 ? w.y : w.x, cr, 0, 0, 0);
+        if (q + 2 < NK) a[(q + 2) % 3] = aread(buf, 0, kstep(q + 2));
+        cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q % 3], ks & 1 ? w.y : w.x, cr, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -261,15 +273,15 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
 #pragma unroll
       for (int lh = 0; lh < 2; ++lh) {
         gd4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
-        double a = aread(buf, lh, 0);
+        double a = aread(buf, lh, kstep(0));
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks) {
-          const int it = lh * NK + ks;
+        for (int q = 0; q < NK; ++q) {
+          const int it = lh * NK + q;
           double2 w;
-          if constexpr (F::RES) w = wb[2 * gr + lh][ks];
+          if constexpr (F::RES) w = wb[2 * gr + lh][kstep(q)];
           else w = bq[it % PD][0];
           double an = 0;
-          if (ks + 1 < NK) an = aread(buf, lh, ks + 1);
+          if (q + 1 < NK) an = aread(buf, lh, kstep(q + 1));
           cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w.x, cr, 0, 0, 0);
           ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w.y, ci, 0, 0, 0);
           if constexpr (!F::RES) {
@@ -284,19 +296,19 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
       }
     } else {
       gd4 c0 = {0, 0, 0, 0}, c1 = {0, 0, 0, 0};
-      double a0 = aread(buf, 0, 0), a1 = aread(buf, 1, 0);
+      double a0 = aread(buf, 0, kstep(0)), a1 = aread(buf, 1, kstep(0));
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) {
-        const int it = ks / 2;
+      for (int q = 0; q < NK; ++q) {
+        const int it = q / 2, ks = kstep(q);
         double2 w0, w1;
-        if constexpr (F::RES) w0 = wb[2 * gr][it], w1 = wb[2 * gr + 1][it];
+        if constexpr (F::RES) w0 = wb[2 * gr][ks / 2], w1 = wb[2 * gr + 1][ks / 2];
         else w0 = bq[it % PD][0], w1 = bq[it % PD][WID - 1];
         double n0 = 0, n1 = 0;
-        if (ks + 1 < NK) n0 = aread(buf, 0, ks + 1), n1 = aread(buf, 1, ks + 1);
+        if (q + 1 < NK) n0 = aread(buf, 0, kstep(q + 1)), n1 = aread(buf, 1, kstep(q + 1));
         c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, ks & 1 ? w0.y : w0.x, c0, 0, 0, 0);
         c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, ks & 1 ? w1.y : w1.x, c1, 0, 0, 0);
         if constexpr (!F::RES) {
-          if (ks & 1) {
+          if (q & 1) {
             if (it + PD < SEQ) bnext(gr, it + PD);
             else bnext(ng, it + PD - SEQ);
           }
@@ -312,8 +324,7 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
     }
   };
 
-  // S-point DFT and stores of a tile, round rd of the exchange: LPW-point DFTs of the wave's lanes
-  // into G, and NW-point DFTs out of G to HBM.  `wait` runs before the first stores.
+  // S-point DFT of a tile, round rd of the exchange: LPW-point DFTs of the wave's lanes into G
   auto put = [&](int rd) __attribute__((always_inline)) {
     int tv = tid;
     asm volatile("" : "+v"(tv));  // keep the addresses below out of registers in the tile loop
@@ -336,6 +347,7 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
       }
     }
   };
+  // ... and NW-point DFTs out of G to HBM.  `wait` runs before the first stores.
   auto get = [&](int rd, long tile, auto wait) __attribute__((always_inline)) {
     const int jrem = (int)min((long)F::TJ, nJ - tile * F::TJ);  // the last tile may hold fewer row groups
     int tv = tid;

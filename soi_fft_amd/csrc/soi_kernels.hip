@@ -23,6 +23,21 @@ using namespace soi;
 // Tables (init only; FP64 on the GPU)
 // =============================================================================================
 
+// sin and cos of pi num/den, the rounding of the quotient made good: a quotient near 1 is off by up to
+// 5e-17, the angle by 1.7e-16, more than the rounding of the entry itself
+__device__ __forceinline__ void sincospi_ratio(long num, long den, double *sn, double *cs)
+{
+  long r = num % (2 * den);
+  if (r < -den) r += 2 * den;
+  else if (r >= den) r -= 2 * den;
+  const double hi = (double)r / (double)den;
+  const double lo = M_PI * (fma(-hi, (double)den, (double)r) / (double)den);
+  double s0, c0;
+  sincospi(hi, &s0, &c0);
+  *sn = fma(c0, lo, s0);
+  *cs = fma(-s0, lo, c0);
+}
+
 // Filter taps and phase factors.  The reference window (pfft.c:42-66) is
 //   w[theta][b][i] = e^{i pi t} y(t) / mu,  t = theta*d/n - b - i/S + kappa/2,
 //   y(t) = sin(pi tau t)/(pi tau t) * exp(-pi^2 t^2 / sigma), y(0) = 1.
@@ -34,6 +49,36 @@ using namespace soi;
 //          post = e^{i pi (theta d/n + kappa/2 - i/S)}.
 // ct = 1: taps[theta][i][b] = w (complex), post = 1.
 // w_full receives w in the reference's logical layout [theta][b][i] (descriptor field w).
+
+// y(t)/mu for t = num/den, rounded once but for sincospi and exp: the values between are sums hi + lo.
+// With t and pi tau t rounded, a tap is off by up to 1e-16 of the largest one whatever its own size:
+// that was over half of the filter's error (S = 4, B = 76: 2.7e-16, with these taps 2.1e-16).
+__device__ __forceinline__ double window_y_mu(long num, long den, double tau, double sigma, double mu)
+{
+  if (num == 0) return __ddiv_rn(1.0, mu);
+  const double PI_LO = 1.2246467991473532e-16;  // pi - M_PI
+  const double t = (double)num / (double)den;
+  const double tl = fma(-t, (double)den, (double)num) / (double)den;
+  // a = tau t, d = pi a
+  const double a = __dmul_rn(tau, t), al = fma(tau, t, -a) + tau * tl;
+  const double d = __dmul_rn(M_PI, a), dl = fma(M_PI, a, -d) + (M_PI * al + PI_LO * a);
+  double s0, c0;
+  sincospi(a, &s0, &c0);
+  const double q = __ddiv_rn(s0, d);  // sin(pi a)/(pi a)
+  const double ql = (fma(-q, d, s0) + (c0 * (M_PI * al) - q * dl)) / d;
+  // g = (pi t)^2 / sigma
+  const double u = __dmul_rn(M_PI, t), ul = fma(M_PI, t, -u) + (M_PI * tl + PI_LO * t);
+  const double v = __dmul_rn(u, u), vl = fma(u, u, -v) + 2 * u * ul;
+  const double g = __ddiv_rn(v, sigma);
+  if (g > 800) return 0.0;
+  const double gl = g == 0 ? 0.0 : (fma(-g, sigma, v) + vl) / sigma;
+  const double e = exp(-g);
+  const double y = __dmul_rn(q, e), yl = fma(q, e, -y) + e * (ql - q * gl);
+  const double r = __ddiv_rn(y, mu);
+  return r + (fma(-r, mu, y) + yl) / mu;
+}
+
+// y(t) as the reference forms it, from a rounded t
 __device__ __forceinline__ double window_y(double t, double tau, double sigma)
 {
   if (t == 0.0) return 1.0;
@@ -64,37 +109,29 @@ __global__ void k_make_taps(void *taps, double2 *post, double2 *w_full, int S, i
   const int kappa = B - d_mu;
   const double mu = (double)n_mu / (double)d_mu;
   long num0 = 2L * theta * d_mu * S + (long)kappa * n_mu * S - 2L * i * n_mu;  // (t + b) * den
-  // post phase e^{i pi num0/den}: num0 reduced modulo 2*den (period 2 in units of pi)
-  long r0 = num0 % (2 * den);
-  if (r0 < 0) r0 += 2 * den;
   double sp0, cp0;
-  sincospi((double)r0 / (double)den, &sp0, &cp0);
+  sincospi_ratio(num0, den, &sp0, &cp0);  // post phase
   if (b == 0) post[theta * S + i] = ct ? double2{1.0, 0.0} : double2{cp0, sp0};
   double2 wv = double2{0.0, 0.0};
   if (b < B) {
-    double t;
-    double sp, cp;
+    double sp, cp, ymu = 0;
     if (ref) {
       long j = (long)b * S + i;
       double a0 = __ddiv_rn((double)theta, (double)Mh);
       double a1 = __ddiv_rn((double)j, (double)N);
       double a2 = __ddiv_rn((double)kappa, (double)(2 * M));
-      t = __dmul_rn(__dadd_rn(__dsub_rn(a0, a1), a2), (double)M);
+      const double t = __dmul_rn(__dadd_rn(__dsub_rn(a0, a1), a2), (double)M);
       sincospi(t, &sp, &cp);
+      const double y = window_y(t, tau, sigma);
+      wv = double2{__ddiv_rn(__dmul_rn(cp, y), mu), __ddiv_rn(__dmul_rn(sp, y), mu)};
     } else {
-      long num = num0 - 2L * b * n_mu * S;
-      t = (double)num / (double)den;
-      long rr = num % (2 * den);
-      if (rr < 0) rr += 2 * den;
-      sincospi((double)rr / (double)den, &sp, &cp);
+      const long num = num0 - 2L * b * n_mu * S;
+      sincospi_ratio(num, den, &sp, &cp);
+      ymu = window_y_mu(num, den, tau, sigma, mu);
+      wv = double2{__dmul_rn(cp, ymu), __dmul_rn(sp, ymu)};
     }
-    double y = window_y(t, tau, sigma);
-    wv = double2{__ddiv_rn(__dmul_rn(cp, y), mu), __ddiv_rn(__dmul_rn(sp, y), mu)};
     if (w_full) w_full[((long)theta * B + b) * S + i] = wv;
-    if (!ct) {
-      double tap = __ddiv_rn(y, mu);
-      ((double *)taps)[idx] = (b & 1) ? -tap : tap;
-    }
+    if (!ct) ((double *)taps)[idx] = (b & 1) ? -ymu : ymu;  // (exact t only)
   } else if (!ct) {
     ((double *)taps)[idx] = 0.0;
   }

@@ -1,0 +1,101 @@
+"""How far the complex128 stages are from the exact result, in isolation, against long double: a form on
+the matrix units or with larger radices is no less accurate than the plain one that it replaced."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpu_util import d2h, to_dev
+
+pytestmark = pytest.mark.gpu
+
+LD = np.longdouble
+PI = LD("3.14159265358979323846264338327950288")
+
+
+def rel_rms(got, ref):
+    e = got.astype(np.clongdouble) - ref
+    return float(np.sqrt((np.abs(e) ** 2).sum() / (np.abs(ref) ** 2).sum()))
+
+
+def cis(num, den):
+    """e^{i pi num/den} of integers"""
+    r = np.asarray(num) % (2 * den)
+    a = PI * np.where(r > den, r - 2 * den, r).astype(LD) / LD(den)
+    return np.cos(a) + 1j * np.sin(a)
+
+
+def exact_filter(x, S, M, n_mu, d_mu, B, tau, sigma, w):
+    """parallel_filter_subsampling in long double, [S][M_hat]: with the window's closed form, or with the
+    table w of complex taps [theta][b][i]"""
+    nJ, mu = M // d_mu, LD(n_mu) / d_mu
+    rows = x.reshape(M, S).astype(np.clongdouble)
+    i = np.arange(S)
+    out = np.zeros((nJ, n_mu, S), np.clongdouble)
+    for th in range(n_mu):
+        for b in range(B):
+            if w is None:
+                num = 2 * th * d_mu * S + (B - d_mu) * n_mu * S - 2 * i * n_mu - 2 * b * n_mu * S
+                t = num.astype(LD) / (2 * n_mu * S)
+                a = PI * LD(tau) * t
+                y = np.where(a == 0, LD(1), np.sin(a) / np.where(a == 0, LD(1), a))
+                wb = cis(num, 2 * n_mu * S) * (y * np.exp(-PI * PI * t * t / LD(sigma)) / mu)
+            else:
+                wb = w[th, b].astype(np.clongdouble)
+            out[:, th, :] += rows[(np.arange(nJ) * d_mu + b) % M] * wb
+    return (out.reshape(nJ * n_mu, S) @ cis(-2 * np.outer(i, i), S)).T
+
+
+WINDOWS = {
+    "b72": dict(window_mode=2),
+    "b76": dict(window_mode=2, B=76, tau=872 / 1024, sigma=313.1715),
+    "b64": dict(window_mode=2, B=64, tau=818 / 1024, sigma=267.4513),
+    "b60": dict(window_mode=2, B=60, tau=0.75, sigma=230.0),
+    "mu87": dict(n_mu=8, d_mu=7, tau=0.7, sigma=360.0),
+    "ct72": dict(window_mode=1),
+    "ct52": dict(B=52, tau=0.6, sigma=180.0),
+    "b44": dict(B=44, tau=0.5, sigma=121.0936),
+    "b30": dict(B=30, tau=0.154, sigma=73.2102363),
+}
+# Error of the VALU form (FP64 FMAs in two slices of real taps, four of complex) on these inputs, 1e-16
+VALU = {
+    "b72": {64: 3.280}, "b64": {64: 3.183}, "b60": {64: 2.935},
+    "b76": {4: 2.529, 16: 2.892, 32: 2.976, 64: 3.172},
+    "mu87": {4: 1.737, 16: 1.990, 32: 2.094, 64: 2.221},
+    "ct72": {4: 1.724, 16: 1.969, 32: 2.065, 64: 2.188},
+    "ct52": {4: 1.978, 16: 2.184, 32: 2.273, 64: 2.393},
+    "b44": {4: 1.506, 16: 1.785, 32: 1.877, 64: 2.024},
+    "b30": {4: 1.594, 16: 1.826, 32: 1.929, 64: 2.069},
+}
+
+
+@pytest.mark.parametrize("name,S", [(n, S) for n, v in VALU.items() for S in v])
+def test_filter_error(soi, torch_cuda, name, S):
+    """The MFMA filter against the error of the VALU form, 3% for what depends on the inputs.  Real taps are
+    judged by the window itself, complex ones (the reference's values) by the descriptor's table."""
+    torch, kw = torch_cuda, WINDOWS[name]
+    n_mu, d_mu, B = kw.get("n_mu", 5), kw.get("d_mu", 4), kw.get("B", 72)
+    M = 1792 if n_mu == 8 else 1600
+    rng = np.random.default_rng(S)
+    x = rng.uniform(-1, 1, M * S) + 1j * rng.uniform(-1, 1, M * S)
+    d = soi.SoiDesc()
+    soi.set_default_soi_descriptor(d)
+    d.N, d.P, d.k = M * S, 4, S // 4
+    for f, v in kw.items():
+        setattr(d, f, v)
+    at = torch.zeros(S * n_mu * M // d_mu, dtype=torch.complex128, device="cuda")
+    d.alpha_tilde = at.data_ptr()
+    soi.init_soi_descriptor(d, S // 4)
+    try:
+        assert soi.filter_form(d) == soi.SOI_FILTER_MFMA_F64
+        w = None if kw.get("window_mode") == 2 else d2h(ctypes.c_void_p(d.w), n_mu * B * S, np.complex128)
+        xt = to_dev(torch, x)
+        torch.cuda.synchronize()
+        soi.parallel_filter_subsampling(d, xt.data_ptr())
+        got = at.cpu().numpy().reshape(S, -1)
+    finally:
+        soi.free_soi_descriptor(d)
+    ref = exact_filter(x, S, M, n_mu, d_mu, B, d.tau, d.sigma, None if w is None else w.reshape(n_mu, B, S))
+    e = rel_rms(got, ref)
+    print(f"case {name} S={S}: {e:.3e}, VALU form {VALU[name][S]}e-16", flush=True)
+    assert e < 1.03e-16 * VALU[name][S]
