@@ -227,8 +227,7 @@ template <int FORM, int R, typename C> __device__ __forceinline__ void dft_as(C 
 // A stage may be a chain of radices that run one after the other in registers: two decimal digits
 // for each, the first in front (20503 = radix 2, then 5, then 3: 30 values, all twiddles of the
 // three stages from the table).  FORM says how twiddles are made and which DFTs are used:
-//   0: powers of a few table reads (complex128, see chain) or every twiddle from the table
-//      (complex64), products of coprime factors without twiddles;
+//   0: see chain; products of coprime factors without twiddles;
 //   2: every twiddle from the table, as soi_common.hpp's LDS transform does.
 // ---------------------------------------------------------------------------------------------
 constexpr int code_prod(int c) { return c < 100 ? c : c % 100 * code_prod(c / 100); }
@@ -343,39 +342,27 @@ __device__ __forceinline__ void exchange(C (&v)[SC::E], unsigned char *lds, int 
 }
 
 constexpr int odd_part(int x) { return x % 2 ? x : odd_part(x / 2); }
-constexpr int bit_len(int x) { return x ? 1 + bit_len(x >> 1) : 0; }
 
 // The radices of CODE on the values v of one butterfly: input k is position j + k*L/R, output k goes to
 // position k*NS of the butterfly's outputs, jm = j % NS.  The first radix R1 of the chain has R/R1
 // butterflies with the same jm; its output k continues, by itself, with jm + k*NS at span NS*R1.
-// Complex128 (FORM 0): the R1 - 1 twiddles w^k of a butterfly come from the log2 R1 table reads
-// w^(2^b): w^k is the product of the powers of k's set bits (at most three extra roundings for R1 =
-// 16), so a thread issues a few loads per butterfly instead of R1 - 1.  Complex64 reads each: the
-// products cost 3 to 5% of the transform's error (N = 2^22: 3.34e-7 against 3.18e-7) for 0 to 8% of its
-// time.
+// Twiddles w^k: complex64 and FORM 2 read each from the table.  Complex128 (FORM 0) reads those with k < 4 or
+// k % 4 == 0 and forms the others as one product of two of them (radix 16: six reads instead of 15); up to
+// radix 8 it reads all, but for 2048 points and more, where the last stage's loads cost 6% of a whole
+// transform (N = 2^27, S = 32; 8% at 2^24, S = 8).  Products of all of k's bits, up to three of them, had
+// cost 4 to 8% of a pass's error (512-point rows 1.98e-16 -> 2.14e-16; now 1.98e-16).
 template <int FORM, int L, int NS, int CODE, typename C>
 __device__ __forceinline__ void chain(C *v, int jm, const C *__restrict__ tw)
 {
   constexpr int R1 = code_first(CODE), REST = code_rest(CODE), M = REST ? code_prod(REST) : 1;
-  constexpr int NBITS = bit_len(R1 - 1), step = L / (NS * R1);
+  constexpr int step = L / (NS * R1);
   C w[R1];
-  if constexpr (NS > 1 && FORM < 2 && sizeof(C) == 16) {
-    C p[NBITS];
-#pragma unroll
-    for (int b = 0; b < NBITS; ++b) p[b] = tw[(jm * step) << b];
+  if constexpr (NS > 1) {
 #pragma unroll
     for (int k = 1; k < R1; ++k) {
-      bool first = true;
-#pragma unroll
-      for (int b = 0; b < NBITS; ++b)
-        if (k & (1 << b)) {
-          w[k] = first ? p[b] : cmul_as<FORM>(w[k], p[b]);
-          first = false;
-        }
+      if (sizeof(C) == 8 || FORM == 2 || (R1 <= 8 && L < 2048) || k % 4 == 0 || k < 4) w[k] = tw[k * jm * step];
+      else w[k] = cmul_as<FORM>(w[k & ~3], w[k & 3]);
     }
-  } else if constexpr (NS > 1) {
-#pragma unroll
-    for (int k = 1; k < R1; ++k) w[k] = tw[k * jm * step];
   }
   C u[R1][M];
 #pragma unroll
@@ -515,9 +502,11 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_cols(
   // reads NC + RL - 1 table pairs instead of NC * RL (FORM 2: unfactored)
   constexpr int RL = SC::at(SC::n - 1), NC = SC::nc(SC::n - 1), NB = SC::nb(SC::n - 1);
   // Complex64 factors it only for n1 = F 2^a, F = 1 and 5; elsewhere that would add to its error (N =
-  // 27*2^17: 3.23e-7, unfactored 3.17e-7, the same time).
+  // 27*2^17: 3.23e-7, unfactored 3.17e-7, the same time).  Complex128 factors it at 2560 points only, one
+  // block a CU, where it costs no accuracy (4.46 ms at N = 2^27, unfactored 4.6 to 4.9); elsewhere the extra
+  // products are 3% of the pass's error for 0 to 4% of the transform's time.
   constexpr int ODD = odd_part(L);
-  constexpr bool FACT = SC::FORM < 2 && (sizeof(C) == 16 || ODD == 1 || ODD == 5);
+  constexpr bool FACT = SC::FORM < 2 && (sizeof(C) == 16 ? L == 2560 : ODD == 1 || ODD == 5);
   const unsigned lmask = (1u << lb1) - 1;
   if (!on) return;  // no barrier follows
   C tc[NC];

@@ -147,20 +147,18 @@ __global__ void k_make_winv(double2 *winv, long M, int kappa, double tau, double
   double t = (double)m / (double)M - 0.5;
   double ss = sqrt(sigma);
   double y = 1.0 / (2.0 * tau) * (erfc(ss * (t - tau / 2)) - erfc(ss * (t + tau / 2)));
-  long r = ((long)kappa * m) % (2 * M);  // angle = -pi * r / M
   double sp, cp;
-  sincospi((double)r / (double)M, &sp, &cp);
+  sincospi_ratio((long)kappa * m, M, &sp, &cp);
   winv[m] = double2{cp / y, -sp / y};
 }
 
-// tw[m] = e^{-2 pi i m / L} for m < n (exact reduction: m/L in [0,1))
+// tw[m] = e^{-2 pi i m mult / L} for m < n
 __global__ void k_make_twiddles(double2 *tw, long n, long L, long mult)
 {
   long m = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (m >= n) return;
-  long e = (m * mult) % L;
   double sp, cp;
-  sincospi(2.0 * (double)e / (double)L, &sp, &cp);
+  sincospi_ratio(2 * (m * mult % L), L, &sp, &cp);
   tw[m] = double2{cp, -sp};
 }
 

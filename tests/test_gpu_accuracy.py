@@ -99,3 +99,55 @@ def test_filter_error(soi, torch_cuda, name, S):
     e = rel_rms(got, ref)
     print(f"case {name} S={S}: {e:.3e}, VALU form {VALU[name][S]}e-16", flush=True)
     assert e < 1.03e-16 * VALU[name][S]
+
+
+class Batch(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_void_p), ("at", ctypes.c_void_p), ("tb", ctypes.c_void_p),
+                ("n", ctypes.c_int)]
+
+
+# Error, 1e-16, of the passes with stages of radix 10 and less or on the LDS kernels, their tables' too
+PASSES = [("cols", 48, 2.067), ("cols", 240, 2.545), ("cols", 480, 2.651), ("rows", 64, 1.526),
+          ("rows", 512, 1.984), ("one", 1152, 2.382), ("one", 1280, 2.276), ("one", 5120, 2.508)]
+
+
+@pytest.mark.parametrize("kind,L,former", PASSES)
+def test_pass_error(soi, torch_cuda, kind, L, former):
+    """A complex128 FFT pass with the library's own twiddle tables against the error of the stages and
+    tables before these, 4% for what depends on the inputs."""
+    import scipy.fft
+    torch, lib, vp, cl = torch_cuda, soi.lib(), ctypes.c_void_p, ctypes.c_long
+
+    def table(n, mult, of):
+        t = torch.zeros(n, dtype=torch.complex128, device="cuda")
+        assert lib.soik_make_twiddles(vp(t.data_ptr()), cl(n), cl(of), cl(mult), None) == 0
+        return t
+
+    p = lambda t: vp(t.data_ptr())
+    b, other, S = Batch(), 40, 4
+    if kind == "one":
+        other, S = 1, 32
+    Mh = L * other
+    rng = np.random.default_rng(L)
+    shape = (S, L, other) if kind == "cols" else (S, other, L)
+    x = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    y = to_dev(torch, x)
+    out = torch.zeros(S * Mh, dtype=torch.complex128, device="cuda")
+    one = torch.ones(Mh, dtype=torch.complex128, device="cuda")
+    tw = table(L, 1, L)
+    print(f"case {kind} L={L}", flush=True)
+    ref = scipy.fft.fft(x.astype(np.clongdouble), axis=1 if kind == "cols" else 2)
+    if kind == "cols":
+        lb = max(6, (Mh - 1).bit_length() // 2)
+        hi, lo = table((Mh >> lb) + 1, 1 << lb, Mh), table(1 << lb, 1, Mh)
+        assert lib.soik_fft_cols(p(y), p(tw), p(hi), p(lo), L, other, lb, cl(Mh), S, 0, None, cl(0), b, None) == 0
+        out, ref = y, ref * cis(-2 * np.outer(np.arange(L), np.arange(other)), Mh)
+    elif kind == "rows":
+        assert lib.soik_fft_rows(p(y), p(out), p(tw), p(one), other, L, cl(Mh), cl(Mh), S, 0, b, None) == 0
+        ref = ref.transpose(0, 2, 1)
+    else:
+        assert lib.soik_fft_one(p(y), p(out), p(tw), p(one), L, cl(L), S, b, None) == 0
+    torch.cuda.synchronize()
+    e = rel_rms(out.cpu().numpy().reshape(ref.shape), ref)
+    print(f"  {e:.3e}, before {former}e-16", flush=True)
+    assert e < 1.04e-16 * former
