@@ -501,12 +501,12 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_cols(
   // lo[e & mask], exponents below M_hat < 2^32), factored into w^{r2 j} w^{r2 k L/RL}: a thread
   // reads NC + RL - 1 table pairs instead of NC * RL (FORM 2: unfactored)
   constexpr int RL = SC::at(SC::n - 1), NC = SC::nc(SC::n - 1), NB = SC::nb(SC::n - 1);
-  // Complex64 factors it only for n1 = F 2^a, F = 1 and 5; elsewhere that would add to its error (N =
+  // Complex64 factors it only for n1 = F 2^a >= 256, F = 1 and 5; elsewhere that would add to its error (N =
   // 27*2^17: 3.23e-7, unfactored 3.17e-7, the same time).  Complex128 factors it at 2560 points only, one
   // block a CU, where it costs no accuracy (4.46 ms at N = 2^27, unfactored 4.6 to 4.9); elsewhere the extra
   // products are 3% of the pass's error for 0 to 4% of the transform's time.
   constexpr int ODD = odd_part(L);
-  constexpr bool FACT = SC::FORM < 2 && (sizeof(C) == 16 ? L == 2560 : ODD == 1 || ODD == 5);
+  constexpr bool FACT = SC::FORM < 2 && (sizeof(C) == 16 ? L == 2560 : L >= 256 && (ODD == 1 || ODD == 5));
   const unsigned lmask = (1u << lb1) - 1;
   if (!on) return;  // no barrier follows
   C tc[NC];

@@ -151,3 +151,28 @@ def test_pass_error(soi, torch_cuda, kind, L, former):
     e = rel_rms(out.cpu().numpy().reshape(ref.shape), ref)
     print(f"  {e:.3e}, before {former}e-16", flush=True)
     assert e < 1.04e-16 * former
+
+
+# Error, 1e-7, of complex64 transforms of uniform noise on the LDS kernels' stages
+SINGLE = [(40960, 8, 2.779), (9 * 2 ** 19, 8, 3.172), (27 * 2 ** 18, 8, 3.170), (27 * 2 ** 18, 32, 3.161),
+          (3 * 2 ** 22, 8, 3.210)]
+
+
+@pytest.mark.parametrize("N,P,former", SINGLE)
+def test_single_precision_error(soi, torch_cuda, N, P, former):
+    """Lengths with odd factors against the error of the kernels before the register passes, 0.5% for
+    what depends on the inputs."""
+    torch = torch_cuda
+    g = torch.Generator(device="cuda").manual_seed(10)
+    x = torch.rand((N, 2), generator=g, device="cuda", dtype=torch.float64).mul_(2).sub_(1)
+    x = torch.view_as_complex(x).to(torch.complex64)
+    ref = torch.fft.fft(x.to(torch.complex128))
+    d = soi.make_descriptor(N, P, precision=soi.SOI_PREC_FP32)
+    try:
+        torch.cuda.synchronize()
+        soi.compute_soi(d, x.data_ptr())
+    finally:
+        soi.free_soi_descriptor(d)
+    e = (torch.linalg.norm(x.to(torch.complex128) - ref) / torch.linalg.norm(ref)).item()
+    print(f"case N={N} P={P}: {e:.4e}, before {former}e-7", flush=True)
+    assert e < 1.005e-7 * former
