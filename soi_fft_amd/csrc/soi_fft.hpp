@@ -346,11 +346,13 @@ constexpr int odd_part(int x) { return x % 2 ? x : odd_part(x / 2); }
 // The radices of CODE on the values v of one butterfly: input k is position j + k*L/R, output k goes to
 // position k*NS of the butterfly's outputs, jm = j % NS.  The first radix R1 of the chain has R/R1
 // butterflies with the same jm; its output k continues, by itself, with jm + k*NS at span NS*R1.
-// Twiddles w^k: complex64 and FORM 2 read each from the table.  Complex128 (FORM 0) reads those with k < 4 or
-// k % 4 == 0 and forms the others as one product of two of them (radix 16: six reads instead of 15); up to
-// radix 8 it reads all, but for 2048 points and more, where the last stage's loads cost 6% of a whole
-// transform (N = 2^27, S = 32; 8% at 2^24, S = 8).  Products of all of k's bits, up to three of them, had
-// cost 4 to 8% of a pass's error (512-point rows 1.98e-16 -> 2.14e-16; now 1.98e-16).
+// Twiddles w^k: FORM 2 reads each from the table.  FORM 0 reads those with k < 4 or k % 4 == 0 and forms the
+// others as one product of two of them (radix 16: six reads instead of 15).  Products of all of k's
+// bits, up to three of them, cost 4 to 8% of a complex128 pass's error (512-point rows 1.98e-16 ->
+// 2.14e-16, now 1.98e-16).  Up to radix 8 complex128 reads all, but for 2048 points and more, where the last
+// stage's loads cost 6% of a whole transform (N = 2^27, S = 32; 8% at 2^24, S = 8).  Complex64 waits for
+// loads more: reading all costs 0 to 8% of a transform (N = 2^23, S = 32 161 -> 167 us, 2^26 1309 -> 1491) for 1 to
+// 4% of its error (3*2^22, S = 8 2.96e-7 -> 2.84e-7).
 template <int FORM, int L, int NS, int CODE, typename C>
 __device__ __forceinline__ void chain(C *v, int jm, const C *__restrict__ tw)
 {
@@ -360,7 +362,7 @@ __device__ __forceinline__ void chain(C *v, int jm, const C *__restrict__ tw)
   if constexpr (NS > 1) {
 #pragma unroll
     for (int k = 1; k < R1; ++k) {
-      if (sizeof(C) == 8 || FORM == 2 || (R1 <= 8 && L < 2048) || k % 4 == 0 || k < 4) w[k] = tw[k * jm * step];
+      if (FORM == 2 || (sizeof(C) == 16 && R1 <= 8 && L < 2048) || k % 4 == 0 || k < 4) w[k] = tw[k * jm * step];
       else w[k] = cmul_as<FORM>(w[k & ~3], w[k & 3]);
     }
   }
