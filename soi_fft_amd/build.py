@@ -20,7 +20,7 @@ ARCH = os.environ.get("SOI_OFFLOAD_ARCH", "gfx950")
 HIP_SOURCES = ["soi_filter.hip", "soi_filter_g54.hip", "soi_filter_g87.hip",
                "soi_filter_grt.hip", "soi_kernels.hip", "soi_fft.hip", "soi_fft_cols64.hip",
                "soi_fft_cols32.hip", "soi_fft_rows64.hip", "soi_fft_rows32.hip",
-               "soi_fft_long32.hip", "soi_fft_long32d.hip"]
+               "soi_fft_long32d.hip"]
 C_SOURCES = ["pfft.c", "compress_host.c", "harness.c"]
 DRIVER = os.path.join(HERE, "soi_test")   # command-line driver (soi_test.c), links the library
 

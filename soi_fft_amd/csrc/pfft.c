@@ -96,8 +96,7 @@ typedef struct {
   void *wt; /* complex64 MFMA filter: bf16 tap pieces */
   /* fft */
   int fft_one;                     /* one pass, one segment per block (fft_single then too) */
-  int fft_long;                    /* complex64 of N >= 2^24: the passes of soi_fft_long32.hip */
-  int fft_longd;                   /* ... of soi_fft_long32d.hip */
+  int fft_chain;                   /* complex64: the passes of soi_fft_long32d.hip */
   int fft_single, single_count, fft_reg;
   int n1, n2, Tc, Tr, B1, lb1;
   int cvar, rvar;                  /* tile alternatives of the column and row pass in use */
@@ -257,108 +256,110 @@ static double pass_cost(long n, int rows, int f32)
   return rows ? (n <= 640 ? 0.98 : n <= 1280 ? 1.12 : 1.2) : n <= 1280 ? 1.0 : 1.16;
 }
 
+/* Split of M_hat for the LDS kernels: n1 x n2, both smooth, column tile Tc >= 2 and row tile Tr >= 2
+ * preferred; minimise max(n1, n2) with n1 a power of two when possible.  0 if there is none. */
+#define LDS_CAP 5120 /* complex values per block: 80 KiB of LDS, two blocks per CU */
+static int lds_split(long Mh, int *n1, int *n2, int *Tc, int *Tr)
+{
+  long best = LONG_MAX;
+  for (long a = 2; a <= LDS_CAP; ++a) {
+    if (Mh % a) continue;
+    const long b = Mh / a;
+    if (b > LDS_CAP || !is_smooth(a) || !is_smooth(b)) continue;
+    const int tc = pick_tile((int)a, b, LDS_CAP), tr = pick_tile((int)b, a, LDS_CAP);
+    if (!tc || !tr) continue;
+    const long cost = (a > b ? a : b) * 4 + (tc < 2) * 100000 + (tr < 2) * 100000 + ((a & (a - 1)) ? 1 : 0);
+    if (cost < best) {
+      best = cost;
+      *n1 = (int)a, *n2 = (int)b, *Tc = tc, *Tr = tr;
+    }
+  }
+  return best < LONG_MAX;
+}
+
+/* Tables and buffers of the split n1 x n2 */
+static void set_split(soi_plan_t *pl, int n1, int n2)
+{
+  int lb = 0;
+  while ((1L << lb) * (1L << lb) < pl->Mh) ++lb;
+  pl->n1 = n1;
+  pl->n2 = n2;
+  pl->B1 = 1 << lb;
+  pl->lb1 = lb;
+  pl->Mt = (long)(n1 + 7) / 8 * 8 * n2;
+}
+
 static int plan_fft(soi_plan_t *pl)
 {
   const long Mh = pl->Mh;
-  const int CAP = 5120; /* complex values per block: 80 KiB of LDS, two blocks per CU */
+  int n1 = 0, n2 = 0, Tc = 0, Tr = 0;
+  /* SOI_FFT_N1 forces the column length of the register passes (tuning) */
+  const char *en = getenv("SOI_FFT_N1");
+  const long force = en ? atol(en) : 0;
   if (!is_smooth(Mh)) {
     set_err(SOI_ERR_ARGS, "M_hat=%ld is not of the form 2^a 3^b 5^c", Mh);
     return -1;
   }
   pl->nvar = 1;
-  pl->fft_long = pl->f32 && pl->N >= 1L << 24;
-  if (!pl->fft_long && Mh < INT_MAX && soik_fft_reg_supported((int)Mh, 2)) {
+  if (Mh < INT_MAX && soik_fft_reg_supported((int)Mh, 2)) {
     pl->fft_single = pl->fft_one = 1;
+    return 0;
+  }
+  /* Complex64 of odd parts other than 1, 5 and 25: chains of small radices where both lengths have them (576
+   * points and more).  Against the passes below, whole transforms over odd factors 3 to 75 and 4 to
+   * 32 segments: N = 2^21 to 2^23.9 5% less on average (0.88 to 1.04 of their time: 3*2^20, S = 4 133 -> 117 us,
+   * 27*2^18, S = 8 208 -> 189, 75*2^16, S = 8 133 -> 138), longer ones 0.92 to 1.02.  They are the only
+   * passes for rows of more than 2560 points. */
+  const int have = lds_split(Mh, &n1, &n2, &Tc, &Tr);
+  long odd = Mh;
+  while (odd % 2 == 0) odd /= 2;
+  if (pl->f32 && !force && have && odd != 1 && odd != 5 && odd != 25 && soik_fft_longd_supported(n1, 0) &&
+      soik_fft_longd_supported(n2, 1)) {
+    pl->fft_chain = pl->fft_reg = 1;
+    set_split(pl, n1, n2);
     return 0;
   }
   /* two register passes: columns of n1 and rows of n2 points that both have kernels.  The split
    * with the least measured pass times, scaled by what is padding in partial column and row tiles;
    * about equal ones by the longer of the two lengths (the shorter it is, the more blocks a CU
-   * holds).  Long complex64 transforms keep their rule: the smallest longer length, then the
-   * longer column. */
+   * holds). */
   {
     double best = 1e300;
-    int bn1 = 0;
-    /* SOI_FFT_N1 forces the column length (tuning) */
-    const char *en = getenv("SOI_FFT_N1");
-    const long force = en ? atol(en) : 0;
-    for (long n1 = 2; n1 <= 2560; ++n1) {
-      if (Mh % n1) continue;
-      const long n2 = Mh / n1;
-      if (n2 > 2560) continue;
-      if (pl->fft_long ? !soik_fft_long32_supported((int)n1) || !soik_fft_long32_supported((int)n2)
-                       : !soik_fft_reg_supported((int)n1, 0) || !soik_fft_reg_supported((int)n2, 1))
-        continue;
-      const long pc = (n2 + 7) / 8 * 8, pr = (n1 + 15) / 16 * 16;
-      const long longer = n1 > n2 ? n1 : n2;
-      double cost = pl->fft_long ? (double)longer
-                                 : pass_cost(n1, 0, pl->f32) * pc / n2 +
-                                       pass_cost(n2, 1, pl->f32) * pr / n1 + 1e-4 * longer;
-      if (force == n1) cost = 0;
-      if (cost < best || (cost == best && pl->fft_long)) {
+    int b1 = 0;
+    for (long a = 2; a <= 2560; ++a) {
+      if (Mh % a) continue;
+      const long b = Mh / a;
+      if (b > 2560 || !soik_fft_reg_supported((int)a, 0) || !soik_fft_reg_supported((int)b, 1)) continue;
+      const long pc = (b + 7) / 8 * 8, pr = (a + 15) / 16 * 16;
+      double cost = pass_cost(a, 0, pl->f32) * pc / b + pass_cost(b, 1, pl->f32) * pr / a + 1e-4 * (a > b ? a : b);
+      if (force == a) cost = 0;
+      if (cost < best) {
         best = cost;
-        bn1 = (int)n1;
+        b1 = (int)a;
       }
     }
-    if (bn1) {
+    if (b1) {
       pl->fft_reg = 1;
-      pl->n1 = bn1;
-      pl->n2 = (int)(Mh / bn1);
-      int lb = 0;
-      while ((1L << lb) * (1L << lb) < Mh) ++lb;
-      pl->B1 = 1 << lb;
-      pl->lb1 = lb;
-      pl->Mt = (long)(pl->n1 + 7) / 8 * 8 * pl->n2;
-      pl->nvar = pl->fft_long ? 1 + (pl->n1 == 2560)
-                              : soik_fft_reg_variants(pl->n1, 0) * soik_fft_reg_variants(pl->n2, 1);
+      set_split(pl, b1, (int)(Mh / b1));
+      pl->nvar = soik_fft_reg_variants(pl->n1, 0) * soik_fft_reg_variants(pl->n2, 1);
       return 0;
     }
   }
-  if (Mh + 1 <= CAP) {
+  if (Mh + 1 <= LDS_CAP) {
     pl->fft_single = 1;
-    pl->single_count = (int)(CAP / (Mh + 1));
+    pl->single_count = (int)(LDS_CAP / (Mh + 1));
     if (pl->single_count > pl->S) pl->single_count = (int)pl->S;
     if (pl->single_count < 1) pl->single_count = 1;
     return 0;
   }
-  /* generic LDS kernels: n1 x n2 = Mh, both smooth, column tile Tc >= 2 and row tile Tr >= 2
-   * preferred; minimise max(n1, n2) with n1 a power of two when possible */
-  long best_cost = LONG_MAX;
-  int bn1 = 0, bn2 = 0, bTc = 0, bTr = 0;
-  for (long n1 = 2; n1 <= CAP; ++n1) {
-    if (Mh % n1) continue;
-    long n2 = Mh / n1;
-    if (n2 > CAP || !is_smooth(n1) || !is_smooth(n2)) continue;
-    int Tc = pick_tile((int)n1, n2, CAP), Tr = pick_tile((int)n2, n1, CAP);
-    if (!Tc || !Tr) continue;
-    long cost = (n1 > n2 ? n1 : n2) * 4 + (Tc < 2) * 100000 + (Tr < 2) * 100000 +
-                ((n1 & (n1 - 1)) ? 1 : 0);
-    if (cost < best_cost) {
-      best_cost = cost;
-      bn1 = (int)n1;
-      bn2 = (int)n2;
-      bTc = Tc;
-      bTr = Tr;
-    }
-  }
-  if (!bn1) {
+  if (!have) {
     set_err(SOI_ERR_ARGS, "M_hat=%ld is too long for the two-pass segment FFT (max %d^2)", Mh,
-            CAP);
+            LDS_CAP);
     return -1;
   }
-  pl->n1 = bn1;
-  pl->n2 = bn2;
-  pl->Tc = bTc;
-  pl->Tr = bTr;
-  int b1 = 1, lb = 0;
-  while ((long)b1 * b1 < Mh) b1 <<= 1, ++lb;
-  pl->B1 = b1;
-  pl->lb1 = lb;
-  if (pl->fft_long && soik_fft_longd_supported(bn1, 0) &&
-      soik_fft_longd_supported(bn2, 1)) {
-    pl->fft_longd = pl->fft_reg = 1;
-    pl->Mt = (long)(pl->n1 + 7) / 8 * 8 * pl->n2;
-  }
+  set_split(pl, n1, n2);
+  pl->Tc = Tc;
+  pl->Tr = Tr;
   return 0;
 }
 
@@ -808,16 +809,11 @@ static int run_fft_f32(soi_desc_t *d, soi_plan_t *pl, soi_c32_t *X, SoiBatch b, 
     else
       KCHK(soik_fft_single_f32(at, X, pl->tw1_32, winv, pl->Mh, pl->M, S, pl->single_count, b, st));
     mark(pl, 3, st);
-  } else if (pl->fft_longd) {
+  } else if (pl->fft_chain) {
     KCHK(soik_fft_longd_cols(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
                              S, tb, pl->Mt, b, st));
     mark(pl, 3, st);
     KCHK(soik_fft_longd_rows(tb, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Mt, pl->M, S, b, st));
-  } else if (pl->fft_long && pl->fft_reg) {
-    KCHK(soik_fft_long32_cols(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
-                              S, pl->cvar, tb, b, st));
-    mark(pl, 3, st);
-    KCHK(soik_fft_long32_rows(tb, X, pl->tw2_32, winv, pl->n1, pl->n2, pl->Mh, pl->M, S, b, st));
   } else if (pl->fft_reg) {
     KCHK(soik_fft_cols_f32(at, pl->tw1_32, pl->thi32, pl->tlo32, pl->n1, pl->n2, pl->lb1, pl->Mh,
                            S, pl->cvar, tb, pl->Mt, b, st));
@@ -1017,7 +1013,7 @@ int soi_set_fft_variant(soi_desc_t *d, int v)
   }
   pl->var = v;
   if (pl->fft_reg) {
-    const int nc = pl->fft_long ? pl->nvar : soik_fft_reg_variants(pl->n1, 0);
+    const int nc = soik_fft_reg_variants(pl->n1, 0);
     pl->cvar = v % nc;
     pl->rvar = v / nc;
   }

@@ -1,10 +1,9 @@
-// soi_fft_long32d.hip -- segment FFT passes of long complex64 transforms (N >= 2^24) whose lengths
-// are not both among those of soi_fft_long32.hip, on the stages of soi_fft.hpp.
+// soi_fft_long32d.hip -- complex64 segment FFT passes in chains of small radices, on the stages of soi_fft.hpp,
+// for lengths whose odd part is not 1, 5 or 25 (the planner's choice: plan_fft in pfft.c).
 //
-// For the reason given in soi_fft_long32.hip the results stay those of the LDS kernels that these
-// replace (k_fft_col, k_fft_row), bit for bit: the same radices in the same order (eights, then 4
-// or 2, then fives, then threes), each twiddle from the table.  What changes is where they run: chains of
-// radices in registers, two exchanges instead of four or five passes over LDS.
+// The results are those of the LDS kernels (k_fft_col, k_fft_row), bit for bit: the same radices in the same
+// order (eights, then 4 or 2, then fives, then threes), each twiddle from the table.  What differs is where
+// they run: chains of radices in registers, two exchanges instead of four or five passes over LDS.
 #include "soi_fft.hpp"
 
 using namespace soi;
@@ -19,7 +18,7 @@ using namespace soi;
   X(2000, 100, 8, 205, 505) X(2048, 64, 8, 8, 804) X(2160, 90, 8, 205, 30303) \
   X(2304, 96, 8, 804, 303) X(2400, 120, 8, 405, 503) X(2560, 80, 8, 8, 805)
 
-// rows beside 2560-point columns
+// rows only: beside long columns
 #define SOI_FFT_LONGD_ROWS(X) \
   X(2880, 72, 8, 8, 50303) X(3072, 64, 8, 8, 80203) X(3200, 80, 8, 8, 20505) \
   X(3456, 72, 8, 8, 2030303) X(3840, 80, 8, 8, 40503)

@@ -96,15 +96,7 @@ int soik_fft_rows_f32(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
                       SoiBatch b, hipStream_t st);
 int soik_fft_one_f32(const soi_c32_t *at, soi_c32_t *X, const soi_c32_t *tw,
                      const soi_c64_t *winv, int L, long M, int S, SoiBatch b, hipStream_t st);
-/* complex64 passes of long transforms (soi_fft_long32.hip) */
-int soik_fft_long32_supported(int L);
-int soik_fft_long32_cols(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi,
-                         const soi_c32_t *tlo, int n1, int n2, int lb1, long Mh, int S, int variant,
-                         soi_c32_t *tout, SoiBatch b, hipStream_t st);
-int soik_fft_long32_rows(const soi_c32_t *data, soi_c32_t *X, const soi_c32_t *tw2,
-                         const soi_c64_t *winv, int n1, int n2, long Mh, long M, int S, SoiBatch b,
-                         hipStream_t st);
-/* ... of lengths outside that file's list (soi_fft_long32d.hip), columns (rows = 0) or rows (1) */
+/* complex64 passes in chains of small radices (soi_fft_long32d.hip), columns (rows = 0) or rows (1) */
 int soik_fft_longd_supported(int L, int rows);
 int soik_fft_longd_cols(soi_c32_t *data, const soi_c32_t *tw1, const soi_c32_t *thi,
                         const soi_c32_t *tlo, int n1, int n2, int lb1, long Mh, int S,
