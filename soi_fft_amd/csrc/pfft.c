@@ -111,6 +111,7 @@ typedef struct {
   soi_c64_t *io;        /* device copy of host-pointer inputs */
   char *hs;             /* pinned ring that pageable memory goes through (host_in, host_out) */
   hipEvent_t hs_ev[HS_SLOTS];
+  int host_called;      /* a host-memory call has been made */
   /* the device buffers the kernels use, kept here as well as in the descriptor fields: a
    * reference-style caller may null or overwrite d->alpha_tilde, d->w and d->W_inv between
    * calls (test.c:406-420), and the plan still reaches and frees what it owns */
@@ -384,7 +385,8 @@ static void free_plan(soi_plan_t *pl)
   (void)hipFree(pl->tlo);
   (void)hipFree(pl->io);
   if (pl->hs) {
-    for (int i = 0; i < HS_SLOTS; ++i) (void)hipEventDestroy(pl->hs_ev[i]);
+    for (int i = 0; i < HS_SLOTS; ++i)
+      if (pl->hs_ev[i]) (void)hipEventDestroy(pl->hs_ev[i]);
     (void)hipHostFree(pl->hs);
   }
   (void)hipFree(pl->tbuf);
@@ -683,10 +685,11 @@ static int is_device_ptr(const void *p) { return mem_kind(p) == MEM_DEVICE; }
 /* Pageable host memory and the device: through a ring of pinned chunks, the processor copying one
  * while a kernel moves the other.  The runtime's own copies of pageable memory do not overlap the
  * two on the way back (16 MiB: 466 us in, 934 out; pinned memory takes 300), and their DMA engine starts
- * late after a kernel.  Whole calls, complex128 (before -> here): N = 2^13 61 -> 42 us, 2^16 150 ->
- * 98, 2^18 460 -> 303, 2^20 1650 -> 1020.  Chunks of 2 MiB take 930 there but a ring of two costs a
- * plan's first call 300 us more to allocate than it saves.  N is a multiple of S >= 4, so sizes are
- * multiples of 16 bytes. */
+ * late after a kernel.  Whole calls, complex128 (the runtime's copies -> here): N = 2^13 61 -> 41 us, 2^16 152
+ * -> 98, 2^18 450 -> 305, 2^20 1620 -> 1010, 2^24 25 -> 15.8 ms; with one thread 2^20 1450.  A plan's first call
+ * pays for the ring: 1060 us at 2^20, 150 at 2^16, but below one chunk that is more than it saves, so such
+ * plans take the ring from their second call on (create, one call, free at N = 2^13: 160 us, 185 with
+ * the ring).  N is a multiple of S >= 4, so sizes are multiples of 16 bytes. */
 static size_t host_chunk(size_t bytes) { return bytes < HS_CHUNK ? bytes : HS_CHUNK; }
 static void copy_part(char *dst, const char *src, size_t n)
 {
@@ -703,24 +706,36 @@ static void copy_part(char *dst, const char *src, size_t n)
     if (at < n) memcpy(dst + at, src + at, n - at < part ? n - at : part);
   }
 }
-/* the ring of a plan; 0 where there is none to be had (the runtime's copies then do) */
+/* the ring of a plan; 0 where the runtime's copies do: none to be had, or too early */
 static int host_ring(soi_plan_t *pl, size_t bytes)
 {
   if (pl->hs) return 1;
   const size_t chunk = host_chunk(bytes);
+  if (bytes < HS_CHUNK && !pl->host_called) {
+    pl->host_called = 1;
+    return 0;
+  }
+  const int ne = bytes > chunk ? HS_SLOTS : 0; /* one chunk needs no events */
   int n = 0;
-  while (n < HS_SLOTS && hipEventCreateWithFlags(&pl->hs_ev[n], hipEventDisableTiming) == hipSuccess) ++n;
-  if (n == HS_SLOTS && hipHostMalloc((void **)&pl->hs, bytes > chunk ? HS_SLOTS * chunk : chunk,
-                                     hipHostMallocDefault) == hipSuccess)
+  while (n < ne && hipEventCreateWithFlags(&pl->hs_ev[n], hipEventDisableTiming) == hipSuccess) ++n;
+  if (n == ne && hipHostMalloc((void **)&pl->hs, ne ? HS_SLOTS * chunk : chunk, hipHostMallocDefault) == hipSuccess)
     return 1;
   pl->hs = NULL;
-  while (n > 0) (void)hipEventDestroy(pl->hs_ev[--n]);
+  while (n > 0) {
+    (void)hipEventDestroy(pl->hs_ev[--n]);
+    pl->hs_ev[n] = NULL;
+  }
   (void)hipGetLastError();
   return 0;
 }
 static int host_in(soi_plan_t *pl, char *dev, const char *src, size_t bytes, hipStream_t st)
 {
   const size_t chunk = host_chunk(bytes);
+  if (bytes <= chunk) {
+    copy_part(pl->hs, src, bytes);
+    KCHK(soik_copy(dev, pl->hs, bytes, st));
+    return 0;
+  }
   for (size_t at = 0, i = 0; at < bytes; at += chunk, ++i) {
     const size_t n = bytes - at < chunk ? bytes - at : chunk;
     char *slot = pl->hs + i % HS_SLOTS * chunk;
@@ -736,6 +751,12 @@ fail:
 static int host_out(soi_plan_t *pl, char *dst, const char *dev, size_t bytes, hipStream_t st)
 {
   const size_t chunk = host_chunk(bytes), nc = (bytes + chunk - 1) / chunk;
+  if (nc == 1) {
+    KCHK(soik_copy(pl->hs, dev, bytes, st));
+    HIPCHK(hipStreamSynchronize(st));
+    copy_part(dst, pl->hs, bytes);
+    return 0;
+  }
   for (size_t i = 0; i < nc + HS_SLOTS; ++i) {
     if (i >= HS_SLOTS && i - HS_SLOTS < nc) { /* chunk i - HS_SLOTS out of its slot */
       const size_t at = (i - HS_SLOTS) * chunk;
