@@ -169,7 +169,8 @@ int soi_last_status(void);
 /* compute_soi on a caller-chosen HIP stream (hipStream_t passed as void*; NULL = the
  * descriptor's own stream) without a final synchronisation: returns after enqueueing when
  * alpha_dt is a device pointer, with use_vlc too (the VLC plan is computed on the device and
- * copied to segmentBoundaries asynchronously). */
+ * copied to segmentBoundaries asynchronously).  With a host pointer it returns when the result is in
+ * place; pageable memory is read once the work before it in the stream is done. */
 void compute_soi_async(soi_desc_t *d, cfft_complex_t *alpha_dt, void *stream);
 
 /* Stream the descriptor's kernels run on (hipStream_t as void*). */

@@ -913,7 +913,12 @@ static void compute_impl(soi_desc_t *d, cfft_complex_t *alpha_dt, void *stream, 
           return;
         }
       }
-      ring = kind == MEM_PAGEABLE && host_ring(pl, bytes);
+      if (kind == MEM_PAGEABLE) {
+        /* what the stream still has to do may write the samples, and they are read from here, by the
+         * runtime's copies of small sizes too */
+        HIPCHK(hipStreamSynchronize(st));
+        ring = host_ring(pl, bytes);
+      }
       if (!ring) HIPCHK(hipMemcpyAsync(pl->io, alpha_dt, bytes, hipMemcpyHostToDevice, st));
       else if (host_in(pl, (char *)pl->io, (const char *)alpha_dt, bytes, st)) return;
       buf = pl->io;

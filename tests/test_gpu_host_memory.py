@@ -39,3 +39,39 @@ def test_host_matches_device(soi, torch_cuda, N, P, single):
         assert np.array_equal(pinned.numpy().view(np.uint8), ref.view(np.uint8))
     finally:
         soi.free_soi_descriptor(d)
+
+
+@pytest.mark.parametrize("N", [2 ** 14, 2 ** 18])
+def test_pageable_memory_is_read_in_stream_order(soi, torch_cuda, N):
+    """A host function on the caller's stream fills the pageable buffer; the transform that follows in the stream
+    reads what it wrote, on a plan's first call and later ones (one chunk and a ring)."""
+    import ctypes
+    import time
+
+    from gpu_util import hip
+    torch = torch_cuda
+    rng = np.random.default_rng(N)
+    x = rng.uniform(-1, 1, N) + 1j * rng.uniform(-1, 1, N)
+    d = soi.make_descriptor(N, 4)
+    t = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    buf = np.zeros_like(x)
+
+    @ctypes.CFUNCTYPE(None, ctypes.c_void_p)
+    def fill(_):
+        time.sleep(0.05)
+        buf[:] = x
+
+    s = torch.cuda.Stream()
+    print(f"case host function N={N}", flush=True)
+    try:
+        soi.compute_soi(d, t.data_ptr())
+        ref = t.cpu().numpy()
+        for _ in range(3):
+            buf[:] = 0
+            assert hip().hipLaunchHostFunc(ctypes.c_void_p(s.cuda_stream), fill, None) == 0
+            soi.compute_soi_async(d, buf.ctypes.data, s.cuda_stream)
+            s.synchronize()
+            assert np.array_equal(buf.view(np.uint8), ref.view(np.uint8))
+    finally:
+        soi.free_soi_descriptor(d)
