@@ -897,15 +897,18 @@ __global__ void k_vlc_plan(const int *__restrict__ exps, int S, int P, int k, lo
       }
       bd[p] = (pcs[lo] - target > target - pcs[lo - 1]) ? lo - 1 : lo;
     }
-  } else if (tid == 0) {  // the reference's walk
+  } else if (tid == 0) {  // the reference's walk, ended at the last segment (ratio negative or NaN)
     int s = 1;
     for (int p = 1; p < P;) {
       const double target = p * costPerRank;
       if (pcs[s] >= target) {
         bd[p] = (pcs[s] - target > target - pcs[s - 1]) ? s - 1 : s;
         ++p;
-      } else {
+      } else if (s < S) {
         ++s;
+      } else {
+        bd[p] = S;
+        ++p;
       }
     }
   }
