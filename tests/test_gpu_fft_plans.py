@@ -78,3 +78,57 @@ def test_chains_whole_transform(soi, torch_cuda, N, P):
     finally:
         for d in descs:
             soi.free_soi_descriptor(d)
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("N,P,alternatives", [(2 ** 24, 8, 2), (2 ** 24, 4, 2), (5 * 2 ** 20, 8, 2), (2 ** 22, 16, 1)])
+def test_every_alternative(soi, torch_cuda, N, P, alternatives, single):
+    """Every alternative tile of a plan (two where a length has more than 640 points, but rows of 2048) against the
+    FP64 DFT, and against alternative 0: the same stages in the same order, so within 1e-15 in
+    complex128 and 1e-6 in complex64."""
+    torch = torch_cuda
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.view_as_complex(torch.rand((N, 2), generator=g, device="cuda", dtype=torch.float64).mul_(2).sub_(1))
+    if single:
+        x = x.to(torch.complex64)
+    ref = dft(torch, x)
+    d = soi.make_descriptor(N, P, precision=soi.SOI_PREC_FP32 if single else soi.SOI_PREC_FP64)
+    try:
+        nv, outs, errs = soi.fft_variants(d), [], []
+        assert nv >= alternatives
+        for v in range(nv):
+            soi.set_fft_variant(d, v)
+            y = x.clone()
+            torch.cuda.synchronize()
+            soi.compute_soi(d, y.data_ptr())
+            errs.append(rel(torch, y, ref))
+            outs.append(y)
+        apart = [rel(torch, y, outs[0].to(torch.complex128)) for y in outs]
+    finally:
+        soi.free_soi_descriptor(d)
+    print(f"case N={N} P={P} single={single}: {errs}, apart {apart}", flush=True)
+    assert max(errs) < (3.5e-7 if single else 3e-14)
+    assert max(apart) < (1e-6 if single else 1e-15)
+
+
+@pytest.mark.parametrize("single", [False, True])
+def test_forced_column_length(soi, torch_cuda, monkeypatch, single):
+    """SOI_FFT_N1 takes another split (other roundings) of the same transform."""
+    torch = torch_cuda
+    N, P = 2 ** 24, 4
+    x = noise(torch, N, 9) if single else noise(torch, N, 9).to(torch.complex128)
+    ref, outs = dft(torch, x), []
+    for n1 in (None, "2048", "2560"):
+        if n1:
+            monkeypatch.setenv("SOI_FFT_N1", n1)
+        d = soi.make_descriptor(N, P, precision=soi.SOI_PREC_FP32 if single else soi.SOI_PREC_FP64)
+        try:
+            y = x.clone()
+            torch.cuda.synchronize()
+            soi.compute_soi(d, y.data_ptr())
+        finally:
+            soi.free_soi_descriptor(d)
+        assert rel(torch, y, ref) < (3.5e-7 if single else 3e-14)
+        outs.append(y)
+    assert not torch.equal(outs[1], outs[2])
+    assert torch.equal(outs[0], outs[1]) or torch.equal(outs[0], outs[2])
