@@ -349,8 +349,9 @@ constexpr int odd_part(int x) { return x % 2 ? x : odd_part(x / 2); }
 // Twiddles w^k: FORM 2 reads each from the table.  FORM 0 reads those with k < 4 or k % 4 == 0 and forms the
 // others as one product of two of them (radix 16: six reads instead of 15).  Products of all of k's
 // bits, up to three of them, cost 4 to 8% of a complex128 pass's error (512-point rows 1.98e-16 ->
-// 2.14e-16, now 1.98e-16).  Up to radix 8 complex128 reads all, but for 2048 points and more, where the last
-// stage's loads cost 6% of a whole transform (N = 2^27, S = 32; 8% at 2^24, S = 8).  Complex64 waits for
+// 2.14e-16, now 1.98e-16).  Complex128 of 2^a < 2048 points reads all up to radix 8 (512-point rows with products
+// of two 2.08e-16); at 2048 those loads cost 6% of a whole transform (N = 2^27, S = 32; 8% at 2^24, S = 8), and
+// other lengths are as close with products (3 to 6% of the time of N = 45*2^16 and 9*2^19).  Complex64 waits for
 // loads more: reading all costs 0 to 8% of a transform (N = 2^23, S = 32 161 -> 167 us, 2^26 1309 -> 1491) for 1 to
 // 4% of its error (3*2^22, S = 8 2.96e-7 -> 2.84e-7).
 template <int FORM, int L, int NS, int CODE, typename C>
@@ -358,11 +359,12 @@ __device__ __forceinline__ void chain(C *v, int jm, const C *__restrict__ tw)
 {
   constexpr int R1 = code_first(CODE), REST = code_rest(CODE), M = REST ? code_prod(REST) : 1;
   constexpr int step = L / (NS * R1);
+  constexpr bool ALL = FORM == 2 || (sizeof(C) == 16 && R1 <= 8 && odd_part(L) == 1 && L < 2048);
   C w[R1];
   if constexpr (NS > 1) {
 #pragma unroll
     for (int k = 1; k < R1; ++k) {
-      if (FORM == 2 || (sizeof(C) == 16 && R1 <= 8 && L < 2048) || k % 4 == 0 || k < 4) w[k] = tw[k * jm * step];
+      if (ALL || k % 4 == 0 || k < 4) w[k] = tw[k * jm * step];
       else w[k] = cmul_as<FORM>(w[k & ~3], w[k & 3]);
     }
   }
@@ -503,12 +505,12 @@ __global__ __launch_bounds__(T *SC::TS, MW) void k_fft_cols(
   // lo[e & mask], exponents below M_hat < 2^32), factored into w^{r2 j} w^{r2 k L/RL}: a thread
   // reads NC + RL - 1 table pairs instead of NC * RL (FORM 2: unfactored)
   constexpr int RL = SC::at(SC::n - 1), NC = SC::nc(SC::n - 1), NB = SC::nb(SC::n - 1);
-  // Complex64 factors it only for n1 = F 2^a >= 256, F = 1 and 5; elsewhere that would add to its error (N =
-  // 27*2^17: 3.23e-7, unfactored 3.17e-7, the same time).  Complex128 factors it at 2560 points only, one
-  // block a CU, where it costs no accuracy (4.46 ms at N = 2^27, unfactored 4.6 to 4.9); elsewhere the extra
-  // products are 3% of the pass's error for 0 to 4% of the transform's time.
+  // Below 256 points the extra products would cost 5 to 8% of the pass's error (complex128, 64 points; unfactored
+  // in as much time); above, 2 to 3% against 2 to 6% of a whole transform's time (N = 45*2^16, S = 8 89.5 us,
+  // unfactored 95.0; 2^22, S = 16 126 and 131.5).  Complex64 of other odd parts than 1 and 5 stays
+  // unfactored: N = 27*2^17 3.23e-7, unfactored 3.17e-7, in the same time.
   constexpr int ODD = odd_part(L);
-  constexpr bool FACT = SC::FORM < 2 && (sizeof(C) == 16 ? L == 2560 : L >= 256 && (ODD == 1 || ODD == 5));
+  constexpr bool FACT = SC::FORM == 0 && L >= 256 && (sizeof(C) == 16 || ODD == 1 || ODD == 5);
   const unsigned lmask = (1u << lb1) - 1;
   if (!on) return;  // no barrier follows
   C tc[NC];
