@@ -22,8 +22,9 @@
 // What bounds it and what the layout follows from.  FP64 MFMA and FP64 FMA have the same peak
 // (78.6 TFLOP/s); the matrix form wins because one 8-byte LDS read per lane feeds one or two products
 // of 1024 FMAs, where the VALU form (soi_filter.hip) reads 16 bytes for about nine FMAs.  The B
-// operands of all lanes (20 or 40 values per lane i) exceed the registers of a CU beyond S = 16
-// (complex taps) or 32 (real), so there they stream from L2 a few K steps ahead; the rows of all lanes
+// operands of a wave's lanes (NK or 2 NK values per lane i) stay in registers where they take 160 or
+// fewer (RES: complex taps S <= 16 with up to 20 K steps and S = 32 with 10; real taps S <= 16, and S = 32 with
+// 20); elsewhere they stream from L2 a few K steps ahead; the rows of all lanes
 // exceed LDS at S = 64, so lanes go through in groups of 16.  Two row buffers alternate, one filling
 // (direct-to-LDS loads) while the other is multiplied; results of all groups stay in registers until
 // the S-point DFT.  Long transforms of S = 32 with resident real taps have four
@@ -79,7 +80,7 @@ template <int S_, int NMU_, int DMU_, int NK_, bool CT_, bool QUAD_ = false> str
   static constexpr int MIN_M = NCHK * RPC;       // rows of a tile's loads wrap at most once
   static_assert(NK % 2 == 0 || CT, "real taps are loaded two K steps at a time");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
-  static_assert(!QUAD || (RES && !CT && S >= 16 && NC == 1), "four buffers");
+  static_assert(!QUAD || (RES && !CT && S == 32 && NC == 1), "four buffers");
 };
 
 // Products and an 8-point DFT with the fused operations spelled out: a tile's results are then the same bit
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(F::T, 2) void k_filter_g(const double2 *__restrict_
   dma(buf0, t0, 0);
   if constexpr (F::QUAD) {
     dma(buf1, t0, 1);
-    dma(buf2, min(t0 + 2 / NGRP * step, t1), 2 % NGRP);
+    dma(buf2, t0, 2);
   }
 
   for (int e = tid; e < S; e += F::T) tw[e] = twS[e];

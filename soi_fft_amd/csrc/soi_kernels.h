@@ -115,6 +115,7 @@ int soik_vlc_plan(const int *exps, int S, int P, int k, long l, long Mh, double 
                   int *out, double *pcs, long *unused, int *nwords, hipStream_t st);
 int soik_vlc_exchange(int *out, long stride, double *x, int len, int nchunk, const int *e_max_dev,
                       const int *emi, hipStream_t st);
+/* the words by themselves (x stays), and decoding them: for the tests */
 int soik_compress_flat(int *out, long stride, const double *x, int len, int nchunk,
                        const int *e_max_dev, const int *emi, const long *unused, hipStream_t st);
 int soik_decompress_flat(double *out, const int *in, long stride, int len, int nchunk,

@@ -941,7 +941,7 @@ extern "C" int soik_vlc_exchange(int *out, long stride, double *x, int len, int 
   return vlc_exchange<true>(out, stride, x, len, nchunk, e_max_dev, emi, st);
 }
 
-// The two halves by themselves: the words (x stays), and decoding them
+// The two halves by themselves, for the tests: the words (x stays), and decoding them
 extern "C" int soik_compress_flat(int *out, long stride, const double *x, int len, int nchunk,
                                   const int *e_max_dev, const int *emi, const long *,
                                   hipStream_t st)
