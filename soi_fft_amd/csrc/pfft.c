@@ -311,11 +311,10 @@ static int plan_fft(soi_plan_t *pl)
    * 32 segments: N = 2^21 to 2^23.9 5% less on average (0.88 to 1.04 of their time: 3*2^20, S = 4 133 -> 117 us,
    * 27*2^18, S = 8 208 -> 189, 75*2^16, S = 8 133 -> 138), longer ones 0.92 to 1.02.  They are the only
    * passes for rows of more than 2560 points. */
-  const int have = lds_split(Mh, &n1, &n2, &Tc, &Tr);
   long odd = Mh;
   while (odd % 2 == 0) odd /= 2;
-  if (pl->f32 && !force && have && odd != 1 && odd != 5 && odd != 25 && soik_fft_longd_supported(n1, 0) &&
-      soik_fft_longd_supported(n2, 1)) {
+  if (pl->f32 && !force && Mh >= 576L * 576 && odd != 1 && odd != 5 && odd != 25 && lds_split(Mh, &n1, &n2, &Tc, &Tr) &&
+      soik_fft_longd_supported(n1, 0) && soik_fft_longd_supported(n2, 1)) {
     pl->fft_chain = pl->fft_reg = 1;
     set_split(pl, n1, n2);
     return 0;
@@ -353,7 +352,7 @@ static int plan_fft(soi_plan_t *pl)
     if (pl->single_count < 1) pl->single_count = 1;
     return 0;
   }
-  if (!have) {
+  if (!lds_split(Mh, &n1, &n2, &Tc, &Tr)) {
     set_err(SOI_ERR_ARGS, "M_hat=%ld is too long for the two-pass segment FFT (max %d^2)", Mh,
             LDS_CAP);
     return -1;
