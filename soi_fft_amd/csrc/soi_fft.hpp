@@ -721,6 +721,11 @@ static int launch_rows(const C *data, C *X, const C *tw, const double2 *winv, in
   // segments together 48 against 57 us one by one where the data stay in the last-level cache
   // (512 x 512, 32 segments); 0.58 against 0.64 ms where W_inv is 64 MB (2560 x 2048); elsewhere
   // one by one (1024 x 1024, 64 segments: 0.46 against 0.51 ms).
+  // Whole transforms with up to 1, 4, 16 and 64 together, 65 shapes (N = 2^18 to 2^27, odd parts 1
+  // and 3, 8 and 32 segments, one with 64, both precisions): no other number takes 3.5% less than
+  // the rule's, but for four shapes below 2^20 points, where fewer together take up to 7.5% less
+  // (complex64, N = 3*2^18, 8 segments: one by one 34.1 against 36.8 us).  One by one takes 3 to 4%
+  // more at 2^27.
   const bool cached = (double)S * Mh * sizeof(C) <= 192e6;
   // (complex64 FORM 2, whose W_inv entries are twice its values: four together, 133 against 144 us
   // at 1024 x 960, 32 segments.)
